@@ -52,15 +52,6 @@ struct RecArgs {
     int per_line;    // tables laid out [n][nlines] per table
 };
 
-// Orders LDS traffic of one wavefront (a wave-local tile written by some lanes
-// and read by others); waves of the block are not synchronised.
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Table access: per-line tables from global memory ([n][nlines], coalesced
 // across lanes); shared tables from the LDS copy of the block's batch entry,
 // which stores only the present tables in the order F, LM, R, MU, NU, pre (the

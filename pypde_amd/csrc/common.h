@@ -32,6 +32,14 @@ inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s);
 
 constexpr int kWave = 64;
 
+// Orders LDS traffic within one wavefront (other waves are not synchronised).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Workgroups are dispatched to the device's 8 XCDs in turn (workgroup i to
 // XCD i mod 8), and each XCD has its own L2.  Renumbering them so that XCD x
 // runs a contiguous range of work items keeps the cache lines that

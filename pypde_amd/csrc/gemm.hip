@@ -44,14 +44,6 @@ namespace pypde {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-// Orders LDS traffic within one wavefront (other waves are not synchronised).
-__device__ __forceinline__ void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Batch index of one operand: entry e is at  (e/d1 % m1)*s1 + (e/d2 % m2)*s2
 // (m = 0 means no modulus).  A plain strided batch is {s, 0, 1, 0, 1, 0}.
 struct BIdx {

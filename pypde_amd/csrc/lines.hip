@@ -11,7 +11,7 @@
 //   coalesce.
 //
 // * Recurrences (four-diagonal LU sweeps, the offset-2 tridiagonal solve, the
-//   Poisson per-line solves, two-/five-band solves, the derivative recurrence):
+//   Poisson per-line solves, two-/five-band solves):
 //   a block stages a panel of W lines into LDS with coalesced accesses (rows of
 //   W adjacent columns for axis 0, whole rows for axis 1) together with the
 //   operator tables.  Every operator here couples only indices of equal
@@ -349,60 +349,133 @@ struct StencilInvOp {
     }
 };
 
+// ---------------------------------------------------------------------------
 // Chebyshev derivative recurrence (differentiate_cheby.f90:28-53), `order`
-// times, optionally after the stencil, then / scale_pow.  The recurrence reads
-// the other parity's input, so one lane does the whole line.
-__device__ __forceinline__ void cheb_deriv_inplace(double* x, int n)
+// times, optionally after the stencil, then / scale_pow:
+//   d_j = d_{j+2} + 2 (j+1) c_{j+1},   d_0 = d_2 / 2 + c_1.
+//
+// Output entries of one parity form one chain of additions whose other operand
+// comes from the input entries of the opposite parity, so two lanes run a line,
+// the even and the odd outputs, in the reference's order of additions (the
+// results are bit-identical).  What bounds one field of a few hundred points is
+// latency: the block's loads, one chain of n / 2 additions, the stores.  So a
+// block takes few lines (W <= 16: a 128 x 128 field is 8 blocks instead of 2),
+// every thread moves elements with eight loads in flight, the division by
+// scale_pow is spread over all threads, and a chain lane reads its next eight
+// inputs before it stores the current eight outputs over entries that the other
+// lane has already read: both lanes of a line are in one wave, whose LDS
+// accesses run in program order.  One lane per line with a load and a division
+// inside the chain took 42 us at 128 x 128.
+struct DerivArgs {
+    LineGeom g;
+    const double* s;  // stencil sub-diagonal, or null
+    int order, pitch;
+    double scale_pow;
+};
+
+constexpr int kDerivU = 8;  // chain steps / loads in flight
+
+// One pass over the line at x (entry k at x[k pitch]), output parity p, both
+// parities' lanes of the wave together.
+__device__ __forceinline__ void deriv_chain(double* x, int pitch, int n, int p)
 {
-    double cn = x[n - 1];
-    x[n - 1] = 0.0;
-    double dp2 = 0.0, dp1;
-    {
-        const double cj = x[n - 2];
-        const double dj = (double)(2 * (n - 1)) * cn;
-        x[n - 2] = dj;
-        dp1 = dj;
-        cn = cj;
+    const bool top = ((n - 1 - p) & 1) == 0;  // this parity holds entry n - 1 (whose result is 0)
+    const int jt = top ? n - 3 : n - 2;       // first output with a term
+    const int steps = jt >= p ? (jt - p) / 2 + 1 : 0;
+    const int nwin = ((n - 2) / 2 + kDerivU) / kDerivU;  // windows, the same for every lane
+    double acc = 0.0, cur[kDerivU], nxt[kDerivU];
+    auto load = [&](int w, double (&v)[kDerivU]) {
+#pragma unroll
+        for (int u = 0; u < kDerivU; ++u) v[u] = x[max(jt - 2 * (w * kDerivU + u) + 1, 0) * pitch];
+    };
+    load(0, cur);
+    for (int w = 0; w < nwin; ++w) {
+        load(w + 1, nxt);
+        wave_lds_sync();
+        double out[kDerivU];
+#pragma unroll
+        for (int u = 0; u < kDerivU; ++u) {
+            const int t = w * kDerivU + u, j = jt - 2 * t;
+            const double prod = (double)(2 * (j + 1)) * cur[u];
+            if (j == 0) acc = acc / 2.0 + cur[u];
+            else acc = (t == 0 && !top) ? prod : acc + prod;
+            out[u] = acc;
+        }
+#pragma unroll
+        for (int u = 0; u < kDerivU; ++u) {
+            const int t = w * kDerivU + u;
+            if (t < steps) x[(jt - 2 * t) * pitch] = out[u];
+            cur[u] = nxt[u];
+        }
+        if (w == 0 && top) x[(n - 1) * pitch] = 0.0;
+        wave_lds_sync();
     }
-    for (int j = n - 3; j >= 1; --j) {
-        const double cj = x[j];
-        const double dj = dp2 + (double)(2 * (j + 1)) * cn;
-        x[j] = dj;
-        dp2 = dp1;
-        dp1 = dj;
-        cn = cj;
-    }
-    x[0] = dp2 / 2.0 + cn;
 }
 
-struct DerivOp {
-    const double* s;
-    int len_in, n, order;
-    double scale_pow;
-    __device__ void load_tables(double* t, int, int tid, int nt) const
-    {
-        if (s) copy_tab(t, s, len_in, tid, nt);
-    }
-    __device__ void operator()(double* x, const double* t, int p, int, int) const
-    {
-        if (p) return;
-        if (s) {
-            const int M = len_in, N = M + 2;
-            for (int i = N - 1; i >= 0; --i) {
-                double y;
-                if (i >= 2) {
-                    const double tt = t[i - 2] * x[i - 2];
-                    y = (i < M) ? tt + x[i] : tt;
-                } else {
-                    y = x[i];
-                }
-                x[i] = y;
-            }
+template <int AXIS>
+__global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
+{
+    extern __shared__ double lds[];
+    const LineGeom& g = a.g;
+    const int W = g.W, n = g.len_out, pitch = a.pitch;
+    const int bpe = (g.nlines + W - 1) / W;
+    const int b = blockIdx.x / bpe;
+    const int l0 = (blockIdx.x - b * bpe) * W;
+    const int nl = min(W, g.nlines - l0);
+    const double* __restrict__ src = g.src + (long long)b * g.src_bs;
+    double* __restrict__ dst = g.dst + (long long)b * g.dst_bs;
+    const int tid = threadIdx.x;
+    // elements e = tid + 256 q of the panel: (k, c) with c fastest along columns
+    // (W a power of two; the last panel's missing columns are clamped and not
+    // stored), k fastest along rows
+    const int lw = 31 - __clz(W);
+    const int total = AXIS == 0 ? n << lw : n * nl;
+    auto split = [&](int e, int& k, int& c) {
+        if (AXIS == 0) { k = e >> lw; c = e & (W - 1); }
+        else { c = e / n; k = e - c * n; }
+    };
+    for (int e0 = tid; e0 < total; e0 += 256 * kDerivU) {
+        double v[kDerivU], v2[kDerivU];
+#pragma unroll
+        for (int u = 0; u < kDerivU; ++u) {
+            int k, c;
+            split(min(e0 + 256 * u, total - 1), k, c);
+            c = min(c, nl - 1);
+            const long long at = AXIS == 0 ? l0 + c : (long long)(l0 + c) * g.src_ld;
+            const long long st = AXIS == 0 ? g.src_ld : 1;
+            v[u] = src[at + min(k, g.len_in - 1) * st];
+            if (a.s) v2[u] = src[at + max(k - 2, 0) * st];
         }
-        for (int o = 0; o < order; ++o) cheb_deriv_inplace(x, n);
-        for (int i = 0; i < n; ++i) x[i] = x[i] / scale_pow;
+#pragma unroll
+        for (int u = 0; u < kDerivU; ++u) {
+            if (e0 + 256 * u >= total) break;
+            int k, c;
+            split(e0 + 256 * u, k, c);
+            double y = v[u];
+            if (a.s && k >= 2) {
+                const double tt = a.s[k - 2] * v2[u];
+                y = k < g.len_in ? tt + v[u] : tt;
+            }
+            lds[k * pitch + c] = y;
+        }
     }
-};
+    __syncthreads();
+    if (tid < 2 * W) {
+        // a lane pair per line: W even lanes, then W odd lanes
+        const int c = min(tid & (W - 1), nl - 1), p = tid / W;
+        for (int o = 0; o < a.order; ++o) deriv_chain(lds + c, pitch, n, p);
+    }
+    __syncthreads();
+    const double sp = a.scale_pow;
+    for (int e = tid; e < total; e += 256) {
+        int k, c;
+        split(e, k, c);
+        if (c >= nl) continue;
+        double y = lds[k * pitch + c];
+        if (sp != 1.0) y = y / sp;
+        dst[AXIS == 0 ? (long long)k * g.dst_ld + l0 + c : (long long)(l0 + c) * g.dst_ld + k] = y;
+    }
+}
 
 // Upper two-band back substitution (twodma.f90:2-25).
 struct TwodmaOp {
@@ -805,8 +878,25 @@ extern "C" int pypde_cheb_deriv(const pypde_lines* in, const double* s, int orde
     const int n = s ? g.len_in + 2 : g.len_in;
     PYPDE_REQUIRE(g.len_out == n, "derivative output length must be %d", n);
     PYPDE_REQUIRE(n >= 3 || order == 0, "derivative needs n >= 3");
-    return launch_lines(g, DerivOp{s, g.len_in, n, order, scale_pow}, s ? g.len_in : 0,
-                        in->lines_per_block, stream, "pypde_cheb_deriv");
+    if (g.nlines == 0 || g.batch == 0) return OK;
+    // lines per block: as many as 64 KB of LDS hold, at most 16
+    g.W = 16;
+    if (in->lines_per_block > 0) {
+        g.W = 1;
+        while (g.W * 2 <= in->lines_per_block && g.W < 16) g.W *= 2;
+    }
+    while (g.W > 1 && ((long long)n * (g.axis == 0 ? g.W : g.W + 1) * 8 > kLdsBudget || g.W / 2 >= g.nlines))
+        g.W /= 2;
+    DerivArgs a{g, s, order, g.axis == 0 ? g.W : g.W | 1, scale_pow};
+    const size_t shmem = (size_t)n * a.pitch * sizeof(double);
+    PYPDE_REQUIRE(shmem <= (size_t)kLdsBudget, "pypde_cheb_deriv: line length %d too long for an LDS panel", n);
+    const long long blocks = (long long)((g.nlines + g.W - 1) / g.W) * g.batch;
+    PYPDE_REQUIRE(blocks < (1LL << 31), "pypde_cheb_deriv: grid too large");
+    if (g.axis == 0)
+        hipLaunchKernelGGL(cheb_deriv_kernel<0>, dim3((unsigned)blocks), dim3(256), shmem, as_stream(stream), a);
+    else
+        hipLaunchKernelGGL(cheb_deriv_kernel<1>, dim3((unsigned)blocks), dim3(256), shmem, as_stream(stream), a);
+    return check_launch("pypde_cheb_deriv");
 }
 
 static int fdma_common(const pypde_lines* in, const double* l, const double* d, const double* u1,

@@ -120,6 +120,26 @@ def test_derivative_bit_exact(amd, axis, key):
         assert np.array_equal(d, ref), k
 
 
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("N,lines,batch", [(5, 1, 1), (6, 3, 2), (18, 16, 1), (33, 17, 3), (34, 40, 1),
+                                           (96, 80, 1), (511, 5, 1), (512, 9, 2), (1100, 3, 1)])
+def test_derivative_panels_bit_exact(amd, axis, N, lines, batch):
+    """The derivative over panels of 16 lines and fewer (partial panels, several
+    batch entries, lengths where a panel holds 16, 8, 4 lines) is the oracle's
+    recurrence bit for bit, first and second order, with and without the stencil."""
+    pypde_amd, ops, torch = amd
+    from oracle import pypde_oracle as o
+    rng = np.random.default_rng(N)
+    for key in ("CH", "CD"):
+        b, ob = pypde_amd.Base(N, key), o.Basis(N, key)
+        M = N if key == "CH" else N - 2
+        v = rng.standard_normal((batch, M, lines) if axis == 0 else (batch, lines, M))
+        for k in (1, 2):
+            d = host(b.derivative(ops.to_dev(v), k, axis=axis, scale_pow=0.3))
+            ref = np.stack([o._along(lambda a: ob.derivative(a, k), x, axis) / 0.3 for x in v])
+            assert np.array_equal(d, ref), (key, k)
+
+
 @pytest.mark.parametrize("N", [16, 64, 256])
 @pytest.mark.parametrize("axis", [0, 1])
 def test_fdma_bit_exact_and_transpose(amd, N, axis):
