@@ -358,66 +358,70 @@ struct StencilInvOp {
 // comes from the input entries of the opposite parity, so two lanes run a line,
 // the even and the odd outputs, in the reference's order of additions (the
 // results are bit-identical).  What bounds one field of a few hundred points is
-// latency: the block's loads, one chain of n / 2 additions, the stores.  So a
-// block takes few lines (W <= 16: a 128 x 128 field is 8 blocks instead of 2),
-// every thread moves elements with eight loads in flight, the division by
-// scale_pow is spread over all threads, and a chain lane reads its next eight
-// inputs before it stores the current eight outputs over entries that the other
-// lane has already read: both lanes of a line are in one wave, whose LDS
-// accesses run in program order.  One lane per line with a load and a division
-// inside the chain took 42 us at 128 x 128.
+// latency: the block's loads, one chain of n / 2 steps, the stores.  So a block
+// takes few lines (W <= 16: a 128 x 128 field is 8 blocks), the products
+// 2 (j+1) c_{j+1} and the division by scale_pow are spread over all threads with
+// eight loads in flight, and a chain step is one LDS read, one addition and one
+// LDS write at offsets known at compile time.  A lane reads its next inputs
+// before it stores the current outputs over entries that the other lane has
+// already read: both lanes of a line are in one wave, whose LDS accesses run in
+// program order.  Measured 7.4 us (columns) and 8.5 us (rows) at 128 x 128, 17.5
+// and 19 us at 512 x 512; with one lane per line and a load, a product and a
+// division in its chain 42 us at 128 x 128, with products and index arithmetic
+// in the two lanes' chains 36 us at 512 x 512.
 struct DerivArgs {
     LineGeom g;
     const double* s;  // stencil sub-diagonal, or null
-    int order, pitch;
+    int order;
     double scale_pow;
 };
 
 constexpr int kDerivU = 8;  // chain steps / loads in flight
 
-// One pass over the line at x (entry k at x[k pitch]), output parity p, both
-// parities' lanes of the wave together.
-__device__ __forceinline__ void deriv_chain(double* x, int pitch, int n, int p)
+// One pass over a line whose entry k, times 2 k for k >= 2, is at x[k P]:
+// outputs of parity p into the same entries, both parities' lanes together.
+// Entries down to x[-2 kDerivU P] may be read (their values are not used).
+template <int P>
+__device__ __forceinline__ void deriv_chain(double* x, int n, int p)
 {
     const bool top = ((n - 1 - p) & 1) == 0;  // this parity holds entry n - 1 (whose result is 0)
     const int jt = top ? n - 3 : n - 2;       // first output with a term
-    const int steps = jt >= p ? (jt - p) / 2 + 1 : 0;
+    const int jl = p ? 1 : 2;                 // last output of the chain (d_0 follows)
     const int nwin = ((n - 2) / 2 + kDerivU) / kDerivU;  // windows, the same for every lane
+    const double c1 = x[P];
     double acc = 0.0, cur[kDerivU], nxt[kDerivU];
-    auto load = [&](int w, double (&v)[kDerivU]) {
+    double* q = x + jt * P;
 #pragma unroll
-        for (int u = 0; u < kDerivU; ++u) v[u] = x[max(jt - 2 * (w * kDerivU + u) + 1, 0) * pitch];
-    };
-    load(0, cur);
-    for (int w = 0; w < nwin; ++w) {
-        load(w + 1, nxt);
-        wave_lds_sync();
-        double out[kDerivU];
+    for (int u = 0; u < kDerivU; ++u) cur[u] = q[(1 - 2 * u) * P];
+    for (int w = 0, j = jt; w < nwin; ++w, j -= 2 * kDerivU, q -= 2 * kDerivU * P) {
+        if (w + 1 < nwin) {
 #pragma unroll
-        for (int u = 0; u < kDerivU; ++u) {
-            const int t = w * kDerivU + u, j = jt - 2 * t;
-            const double prod = (double)(2 * (j + 1)) * cur[u];
-            if (j == 0) acc = acc / 2.0 + cur[u];
-            else acc = (t == 0 && !top) ? prod : acc + prod;
-            out[u] = acc;
+            for (int u = 0; u < kDerivU; ++u) nxt[u] = q[(1 - 2 * (kDerivU + u)) * P];
         }
+        wave_lds_sync();
 #pragma unroll
         for (int u = 0; u < kDerivU; ++u) {
-            const int t = w * kDerivU + u;
-            if (t < steps) x[(jt - 2 * t) * pitch] = out[u];
+            if (j - 2 * u >= jl) {
+                acc = acc + cur[u];
+                q[-2 * u * P] = acc;
+            }
             cur[u] = nxt[u];
         }
-        if (w == 0 && top) x[(n - 1) * pitch] = 0.0;
-        wave_lds_sync();
     }
+    if (top) x[(n - 1) * P] = 0.0;
+    if (p == 0) x[0] = acc / 2.0 + c1;
+    wave_lds_sync();
 }
 
-template <int AXIS>
+template <int AXIS, int W>
 __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
 {
-    extern __shared__ double lds[];
+    // along rows an odd pitch: neighbouring entries of a line in other banks
+    constexpr int P = AXIS == 0 ? W : (W | 1);
+    extern __shared__ double lds_raw[];
+    double* lds = lds_raw + 2 * kDerivU * P;
     const LineGeom& g = a.g;
-    const int W = g.W, n = g.len_out, pitch = a.pitch;
+    const int n = g.len_out;
     const int bpe = (g.nlines + W - 1) / W;
     const int b = blockIdx.x / bpe;
     const int l0 = (blockIdx.x - b * bpe) * W;
@@ -426,12 +430,11 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
     double* __restrict__ dst = g.dst + (long long)b * g.dst_bs;
     const int tid = threadIdx.x;
     // elements e = tid + 256 q of the panel: (k, c) with c fastest along columns
-    // (W a power of two; the last panel's missing columns are clamped and not
-    // stored), k fastest along rows
-    const int lw = 31 - __clz(W);
-    const int total = AXIS == 0 ? n << lw : n * nl;
+    // (the last panel's missing columns are clamped and not stored), k fastest
+    // along rows
+    const int total = AXIS == 0 ? n * W : n * nl;
     auto split = [&](int e, int& k, int& c) {
-        if (AXIS == 0) { k = e >> lw; c = e & (W - 1); }
+        if (AXIS == 0) { k = e / W; c = e % W; }
         else { c = e / n; k = e - c * n; }
     };
     for (int e0 = tid; e0 < total; e0 += 256 * kDerivU) {
@@ -456,14 +459,22 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
                 const double tt = a.s[k - 2] * v2[u];
                 y = k < g.len_in ? tt + v[u] : tt;
             }
-            lds[k * pitch + c] = y;
+            if (a.order > 0 && k >= 2) y = (double)(2 * k) * y;
+            lds[k * P + c] = y;
         }
     }
-    __syncthreads();
-    if (tid < 2 * W) {
-        // a lane pair per line: W even lanes, then W odd lanes
-        const int c = min(tid & (W - 1), nl - 1), p = tid / W;
-        for (int o = 0; o < a.order; ++o) deriv_chain(lds + c, pitch, n, p);
+    for (int o = 0; o < a.order; ++o) {
+        __syncthreads();
+        if (o > 0) {
+            for (int e = tid; e < n * W; e += 256) {
+                const int k = e / W, c = e % W;
+                if (k >= 2) lds[k * P + c] = (double)(2 * k) * lds[k * P + c];
+            }
+            __syncthreads();
+        }
+        // a lane pair per line: W even lanes, then W odd lanes (lanes past the
+        // last line repeat it)
+        if (tid < 2 * W) deriv_chain<P>(lds + min(tid % W, nl - 1), n, tid / W);
     }
     __syncthreads();
     const double sp = a.scale_pow;
@@ -471,10 +482,24 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
         int k, c;
         split(e, k, c);
         if (c >= nl) continue;
-        double y = lds[k * pitch + c];
+        double y = lds[k * P + c];
         if (sp != 1.0) y = y / sp;
         dst[AXIS == 0 ? (long long)k * g.dst_ld + l0 + c : (long long)(l0 + c) * g.dst_ld + k] = y;
     }
+}
+
+template <int W>
+static size_t deriv_lds(int axis, int n)
+{
+    return (size_t)(n + 2 * kDerivU) * (axis == 0 ? W : (W | 1)) * sizeof(double);
+}
+
+template <int W>
+static void launch_deriv(const DerivArgs& a, unsigned blocks, hipStream_t s)
+{
+    const size_t shmem = deriv_lds<W>(a.g.axis, a.g.len_out);
+    if (a.g.axis == 0) hipLaunchKernelGGL((cheb_deriv_kernel<0, W>), dim3(blocks), dim3(256), shmem, s, a);
+    else hipLaunchKernelGGL((cheb_deriv_kernel<1, W>), dim3(blocks), dim3(256), shmem, s, a);
 }
 
 // Upper two-band back substitution (twodma.f90:2-25).
@@ -879,23 +904,23 @@ extern "C" int pypde_cheb_deriv(const pypde_lines* in, const double* s, int orde
     PYPDE_REQUIRE(g.len_out == n, "derivative output length must be %d", n);
     PYPDE_REQUIRE(n >= 3 || order == 0, "derivative needs n >= 3");
     if (g.nlines == 0 || g.batch == 0) return OK;
-    // lines per block: as many as 64 KB of LDS hold, at most 16
-    g.W = 16;
-    if (in->lines_per_block > 0) {
-        g.W = 1;
-        while (g.W * 2 <= in->lines_per_block && g.W < 16) g.W *= 2;
-    }
-    while (g.W > 1 && ((long long)n * (g.axis == 0 ? g.W : g.W + 1) * 8 > kLdsBudget || g.W / 2 >= g.nlines))
-        g.W /= 2;
-    DerivArgs a{g, s, order, g.axis == 0 ? g.W : g.W | 1, scale_pow};
-    const size_t shmem = (size_t)n * a.pitch * sizeof(double);
-    PYPDE_REQUIRE(shmem <= (size_t)kLdsBudget, "pypde_cheb_deriv: line length %d too long for an LDS panel", n);
+    // lines per block: as many as 64 KB of LDS hold (or the hint), at most 16
+    const int cap = in->lines_per_block > 0 ? in->lines_per_block : 16;
+    auto fits = [&](int w, size_t bytes) { return w <= cap && (w == 1 || w / 2 < g.nlines) && bytes <= (size_t)kLdsBudget; };
+    g.W = fits(16, deriv_lds<16>(g.axis, n)) ? 16 : fits(8, deriv_lds<8>(g.axis, n)) ? 8
+        : fits(4, deriv_lds<4>(g.axis, n)) ? 4 : fits(2, deriv_lds<2>(g.axis, n)) ? 2 : 1;
+    PYPDE_REQUIRE(g.W > 1 || deriv_lds<1>(g.axis, n) <= (size_t)kLdsBudget + 2 * kDerivU * sizeof(double),
+                  "pypde_cheb_deriv: line length %d too long for an LDS panel", n);
     const long long blocks = (long long)((g.nlines + g.W - 1) / g.W) * g.batch;
     PYPDE_REQUIRE(blocks < (1LL << 31), "pypde_cheb_deriv: grid too large");
-    if (g.axis == 0)
-        hipLaunchKernelGGL(cheb_deriv_kernel<0>, dim3((unsigned)blocks), dim3(256), shmem, as_stream(stream), a);
-    else
-        hipLaunchKernelGGL(cheb_deriv_kernel<1>, dim3((unsigned)blocks), dim3(256), shmem, as_stream(stream), a);
+    const DerivArgs a{g, s, order, scale_pow};
+    switch (g.W) {
+    case 16: launch_deriv<16>(a, (unsigned)blocks, as_stream(stream)); break;
+    case 8: launch_deriv<8>(a, (unsigned)blocks, as_stream(stream)); break;
+    case 4: launch_deriv<4>(a, (unsigned)blocks, as_stream(stream)); break;
+    case 2: launch_deriv<2>(a, (unsigned)blocks, as_stream(stream)); break;
+    default: launch_deriv<1>(a, (unsigned)blocks, as_stream(stream)); break;
+    }
     return check_launch("pypde_cheb_deriv");
 }
 
