@@ -656,7 +656,7 @@ def gemm_variants():
     out = {}
     for l in eng.launches:
         for p in ([l.group] if isinstance(l, _SplitRhs) else [l]):
-            if isinstance(p, _GemmGroup):
+            if isinstance(p, _GemmGroup) and p.members:
                 descs = [GemmDesc.from_buffer_copy(m.desc) for m in p.members]
             elif isinstance(p, _Gemm) and p.desc.fold == 0:
                 descs = [GemmDesc.from_buffer_copy(p.desc)]

@@ -351,6 +351,55 @@ typedef struct pypde_rbc_rhs {
 
 int pypde_rbc_rhs_banded(const pypde_rbc_rhs* args, void* stream);
 
+/* One stage of the fused step in eight launches (pypde_rbc_phase), each a set of
+ * independent blocks that hold whole lines of one axis; the phases of a stage run
+ * in order on one stream.  State and workspace are row-major per instance b and
+ * field f; E = 3 b + f.  H0, H1 = (L0 + 1) / 2, (L1 + 1) / 2.
+ *   1  Y1[E][value | d/dx][L0][M1] from X; with rhs also R (pypde_rbc_rhs_banded)
+ *   2  Pr[E][sum | difference over the mirrored y points][L0][H1], the convective
+ *      products (with ratio times the products with the previous stage's
+ *      velocities uv[b][u | v][point | mirror][L0][H1], which it replaces)
+ *   3  Z[E][L0][M1] = mdtb_b Pr BF_y^T
+ *   4  R = Hx^-1 (R + BF_x Z)
+ *   5  X = R Hy^-T;  W2[b][0] = U (H S)^T, W2[b][1] = V (H D S)^T, W2v = V (D S)^T
+ *   6  RP = Poisson lines of (B D S)_x W2[b][0] + (B S)_x W2[b][1];
+ *      div = (D S)_x U S_y^T + S_x W2v
+ *   7  P = RP Q^T with P[0,0] = 0;  W1[b] = RP [T S Q ; T D S Q]^T
+ *   8  U -= (T D S)_x W1[b][0], V -= (T S)_x W1[b][1];
+ *      pres = (pres - nu div beta) + idta S_x P S_y^T
+ * (S: stencils, T = (S^T S)^-1 S^T, D: derivative / scale, H, Q: the Poisson
+ * transforms).  Replaces navier/rbc2d.py:213-434 for one stage.
+ *
+ * Operators are packed for the FP64 MFMA: op[tile][chunk][64][4], lane l and step s
+ * holding A[16 tile + l % 16][16 chunk + 8 (s / 2) + 2 (l / 16) + s % 2], zero past A's
+ * ends, where A's rows are outputs and its columns terms (of one mode parity where noted):
+ *   gx   [U,V | T][value | d/dx][even | odd modes] of the first H0 x points
+ *   gy   [value | d/dy][even | odd modes] of the first H1 y points
+ *   bfy, bfx  [even | odd output modes] over the first H1, H0 points
+ *   wy   H S_y, H (D S)_y, (D S)_y        qy  Q, T S_y Q, T (D S)_y Q (tiles of each in turn)
+ *   cdx  (D S)_x [even | odd output modes] over the modes of the other parity
+ *   corr (T D S)_x [even | odd output modes] over the other parity, (T S)_x over
+ *        the same parity
+ * bds [8][M0]: diagonals -1, 1, 3, 5 of (B D S)_x and -2, 0, 2, 4 of (B S)_x; sn: the
+ * potential's stencil sub-diagonals, M0 of x then M1 of y; dtbc [L0][L1].  Line
+ * solves (see pypde_recurrence) as parity chains padded with zeros to 16 C positions,
+ * C = 2, 4, 8 or 16, the smallest with 16 C >= (M + 1) / 2: hx, hy per E
+ * [even | odd][LM | R | MU | NU][16 C]; prec [even | odd][LM | R | MU | NU][M1][16 C].
+ * mdtb, idta, nu per instance.
+ * Limits: 6 <= M0, M1 <= PYPDE_STAGE_MAX_MODES. */
+#define PYPDE_STAGE_MAX_MODES 512
+typedef struct pypde_rbc_stage {
+    double *X, *pres, *P;
+    double *Y1, *Pr, *Z, *R, *W2, *W2v, *RP, *W1, *div, *uv;
+    const double *gx, *gy, *bfy, *bfx, *wy, *qy, *cdx, *corr;
+    const double *bds, *sn, *dtbc, *hx, *hy, *prec, *mdtb, *idta, *nu;
+    double beta, ratio;
+    int N0, N1, M0, M1, L0, L1, batch;
+} pypde_rbc_stage;
+
+/* phase 1..8; rhs only with phase 1 (or NULL; rows_per_thread must be 1) */
+int pypde_rbc_phase(const pypde_rbc_stage* stage, const pypde_rbc_rhs* rhs, int phase, void* stream);
+
 /* pypde_rbc_products_yfold and pypde_rbc_rhs_banded (one output per thread:
  * rhs->rows_per_thread must be 1) in one launch.  The two are independent --
  * the products read the dealiased fields, the right-hand side the state -- so
@@ -466,6 +515,8 @@ int pypde_plan_add_splitk_reduce(pypde_plan* p, const double* W, int S, const do
                                  const double* X, int xm, int xr, double* C, long long mn,
                                  int entries);
 int pypde_plan_add_rhs_banded(pypde_plan* p, const pypde_rbc_rhs* args);
+int pypde_plan_add_phase(pypde_plan* p, const pypde_rbc_stage* stage, const pypde_rbc_rhs* rhs,
+                         int phase);
 int pypde_plan_add_products_rhs(pypde_plan* p, const double* Y, const double* Yold,
                                 const double* dtbc, double* P, int L0, int L1,
                                 double sign_value, double sign_dy, double ratio, int batch,

@@ -73,6 +73,17 @@ class RbcRhs(ctypes.Structure):
                 ("N1", ctypes.c_int), ("batch", ctypes.c_int), ("rows_per_thread", ctypes.c_int)]
 
 
+class RbcStage(ctypes.Structure):
+    """Mirror of `pypde_rbc_stage`."""
+
+    _fields_ = ([(n, ctypes.c_void_p) for n in
+                 ("X", "pres", "P", "Y1", "Pr", "Z", "R", "W2", "W2v", "RP", "W1", "div", "uv",
+                  "gx", "gy", "bfy", "bfx", "wy", "qy", "cdx", "corr", "bds", "sn", "dtbc", "hx",
+                  "hy", "prec", "mdtb", "idta", "nu")] +
+                [("beta", ctypes.c_double), ("ratio", ctypes.c_double)] +
+                [(n, ctypes.c_int) for n in ("N0", "N1", "M0", "M1", "L0", "L1", "batch")])
+
+
 class MultiInfo(ctypes.Structure):
     """Mirror of `pypde_multi_info`."""
 
@@ -141,6 +152,8 @@ _SIGS = {
     "pypde_plan_add_fdma": ([_vp, _lp, _vp, _vp, _vp, _vp, ctypes.c_longlong], _i),
     "pypde_plan_add_poisson": ([_vp, _lp, _vp, _vp, _i], _i),
     "pypde_rbc_rhs_banded": ([ctypes.c_void_p, _vp], _i),
+    "pypde_rbc_phase": ([ctypes.c_void_p, ctypes.c_void_p, _i, _vp], _i),
+    "pypde_plan_add_phase": ([_vp, ctypes.c_void_p, ctypes.c_void_p, _i], _i),
     "pypde_rbc_products_rhs": ([_vp, _vp, _vp, _vp, _i, _i, _d, _d, _d, _i, ctypes.c_void_p,
                                 _vp], _i),
     "pypde_plan_add_products_rhs": ([_vp, _vp, _vp, _vp, _vp, _i, _i, _d, _d, _d, _i,

@@ -20,14 +20,17 @@ namespace pypde {
 
 enum PlanOpKind { OP_GEMM, OP_GROUPED, OP_RECURRENCE, OP_PRODUCTS, OP_PRODUCTS_YFOLD, OP_REDUCE,
                   OP_RHS_BANDED, OP_FDMA, OP_POISSON, OP_MULTI, OP_AXPBY, OP_TRANSPOSE,
-                  OP_SCALED_SUB, OP_SET_ENTRIES, OP_PRODUCTS_VJP, OP_PRODUCTS_RHS };
+                  OP_SCALED_SUB, OP_SET_ENTRIES, OP_PRODUCTS_VJP, OP_PRODUCTS_RHS, OP_PHASE };
 
 struct PlanOp {
     PlanOpKind kind;
     std::vector<pypde_gemm_desc> descs;  // OP_GEMM (one) / OP_GROUPED (count)
     pypde_lines lines;                   // OP_RECURRENCE
     pypde_recurrence rec;
-    pypde_rbc_rhs rhs;                   // OP_RHS_BANDED
+    pypde_rbc_rhs rhs;                   // OP_RHS_BANDED, OP_PRODUCTS_RHS, OP_PHASE
+    pypde_rbc_stage stage;               // OP_PHASE
+    int phase;
+    bool has_rhs;
     const double* tab[4];                // OP_FDMA: l, d, u1, u2; OP_POISSON: tab, (sing)
     const int* sing;
     long long table_bs;
@@ -87,6 +90,30 @@ static void relocate_desc(const pypde_plan* pl, const intptr_t* dl, pypde_gemm_d
     d.B1 = relocate(pl, dl, d.B1);
 }
 
+static pypde_rbc_rhs relocate_rhs(const pypde_plan* pl, const intptr_t* dl, pypde_rbc_rhs a)
+{
+    a.X = relocate(pl, dl, a.X);
+    a.pres = relocate(pl, dl, a.pres);
+    a.cst = relocate(pl, dl, a.cst);
+    a.R = relocate(pl, dl, a.R);
+    a.mdta = relocate(pl, dl, a.mdta);
+    a.dta = relocate(pl, dl, a.dta);
+    a.fdiff = relocate(pl, dl, a.fdiff);
+    a.tx = relocate(pl, dl, a.tx);
+    a.ty = relocate(pl, dl, a.ty);
+    return a;
+}
+
+static pypde_rbc_stage relocate_stage(const pypde_plan* pl, const intptr_t* dl, pypde_rbc_stage a)
+{
+    for (double** p : {&a.X, &a.pres, &a.P, &a.Y1, &a.Pr, &a.Z, &a.R, &a.W2, &a.W2v, &a.RP, &a.W1, &a.div, &a.uv})
+        *p = relocate(pl, dl, *p);
+    for (const double** p : {&a.gx, &a.gy, &a.bfy, &a.bfx, &a.wy, &a.qy, &a.cdx, &a.corr, &a.bds, &a.sn, &a.dtbc,
+                             &a.hx, &a.hy, &a.prec, &a.mdtb, &a.idta, &a.nu})
+        *p = relocate(pl, dl, *p);
+    return a;
+}
+
 static int run_op(const pypde_plan* pl, const intptr_t* dl, bool moved,
                   const PlanOp& op, void* stream)
 {
@@ -131,21 +158,18 @@ static int run_op(const pypde_plan* pl, const intptr_t* dl, bool moved,
                                         stream);
     case OP_RHS_BANDED:
     case OP_PRODUCTS_RHS: {
-        pypde_rbc_rhs a = op.rhs;
-        a.X = relocate(pl, dl, a.X);
-        a.pres = relocate(pl, dl, a.pres);
-        a.cst = relocate(pl, dl, a.cst);
-        a.R = relocate(pl, dl, a.R);
-        a.mdta = relocate(pl, dl, a.mdta);
-        a.dta = relocate(pl, dl, a.dta);
-        a.fdiff = relocate(pl, dl, a.fdiff);
-        a.tx = relocate(pl, dl, a.tx);
-        a.ty = relocate(pl, dl, a.ty);
+        const pypde_rbc_rhs a = relocate_rhs(pl, dl, op.rhs);
         if (op.kind == OP_RHS_BANDED) return pypde_rbc_rhs_banded(&a, stream);
         return pypde_rbc_products_rhs(relocate(pl, dl, op.p0), relocate(pl, dl, op.p1),
                                       relocate(pl, dl, op.p2), relocate(pl, dl, op.p3), op.L0,
                                       op.L1, op.sign_value, op.sign_dy, op.ratio, op.batch, &a,
                                       stream);
+    }
+    case OP_PHASE: {
+        if (!moved) return pypde_rbc_phase(&op.stage, op.has_rhs ? &op.rhs : nullptr, op.phase, stream);
+        const pypde_rbc_stage st = relocate_stage(pl, dl, op.stage);
+        const pypde_rbc_rhs a = relocate_rhs(pl, dl, op.rhs);
+        return pypde_rbc_phase(&st, op.has_rhs ? &a : nullptr, op.phase, stream);
     }
     case OP_FDMA: {
         pypde_lines g = op.lines;
@@ -340,6 +364,19 @@ extern "C" int pypde_plan_add_rhs_banded(pypde_plan* p, const pypde_rbc_rhs* arg
     PlanOp op{};
     op.kind = OP_RHS_BANDED;
     op.rhs = *args;
+    return add_op(p, std::move(op));
+}
+
+extern "C" int pypde_plan_add_phase(pypde_plan* p, const pypde_rbc_stage* stage, const pypde_rbc_rhs* rhs,
+                                    int phase)
+{
+    PYPDE_REQUIRE(p && stage, "null argument");
+    PlanOp op{};
+    op.kind = OP_PHASE;
+    op.stage = *stage;
+    op.has_rhs = rhs != nullptr;
+    if (rhs) op.rhs = *rhs;
+    op.phase = phase;
     return add_op(p, std::move(op));
 }
 

@@ -1,13 +1,17 @@
 """Fused RBC2D time step on the GPU: a batch of same-shape instances with
 per-instance Rayleigh / Prandtl numbers and time steps.
 
-The Euler IMEX step of navier/rbc2d.py:396-434 is regrouped into 19 kernel
-launches whatever the batch size: every separable 1-D operator chain of the
-reference (stencil -> derivative -> zero-pad -> DCT, forward DCT -> truncate ->
-pseudo-inverse B, ...) is folded into one dense operator per axis and applied
-as a batched MFMA GEMM; the Helmholtz and Poisson solves stay banded line
-solves with the reference's LU factors; the convective products and the
-pressure update are pointwise kernels.
+The Euler IMEX step of navier/rbc2d.py:396-434 is regrouped into eight kernel
+launches per stage whatever the batch size (RBCBatch._phase_launches, csrc/stage.hip):
+every separable 1-D operator chain of the reference (stencil -> derivative ->
+zero-pad -> DCT, forward DCT -> truncate -> pseudo-inverse B, ...) is folded into
+one dense operator per axis, applied on the FP64 matrix cores by parity or mirror
+halves; the Helmholtz and Poisson solves stay banded line solves with the
+reference's LU factors, in the launches of the products next to them.
+
+The step with one launch per operator (below, 17 or so launches) remains for
+exact_solves, for more modes per axis than a phase's lines hold, and as the
+member launches of a heterogeneous batch (group_launches=False).
 
 Data layout in HBM (float64, row-major):
   X    [B, 3, M0, M1]      Galerkin coefficients of U, V (ChebDirichlet^2) and
@@ -39,7 +43,7 @@ import numpy as np
 import torch
 
 from . import ops
-from ._lib import BIdx, GemmDesc, Lines, RbcRhs, check, lib
+from ._lib import BIdx, GemmDesc, Lines, RbcRhs, RbcStage, check, lib
 from .bases import Base, cheb_backward_matrix, cheb_forward_matrix, pseudoinverse_d2
 from ._lib import Recurrence
 from .solver import (fdma_lu, poisson_line_tables, rec_from_fdma, rec_from_poisson,
@@ -233,6 +237,54 @@ class _GemmGroup:
               self.name)
 
 
+class _Phase(_GemmGroup):
+    """One phase of a stage (pypde_rbc_phase): the phase's independent products
+    and line solves in one launch.  Its tiling follows from the sizes alone."""
+
+    def __init__(self, name, stage, rhs, phase, flops):
+        self.name, self.flops, self.members, self.split = name, flops, [], False
+        self.fn = lib.pypde_rbc_phase
+        self.args = (ctypes.byref(stage), ctypes.byref(rhs) if rhs is not None else None, phase)
+
+    @property
+    def variant(self):
+        return self.args[2]
+
+    def __call__(self, stream):
+        check(self.fn(*self.args, stream), self.name)
+
+
+def pack_operator(A, tiles=None, chunks=None):
+    """A [outputs, terms] in the order the FP64 MFMA consumes it, op[tile][chunk][64][4]
+    (include/pypde_amd.h, pypde_rbc_stage), zero-padded to the given tiles and chunks."""
+    A = np.asarray(A, dtype=float)
+    t = -(-A.shape[0] // 16) if tiles is None else tiles
+    c = -(-A.shape[1] // 16) if chunks is None else chunks
+    out = np.zeros((16 * t, 16 * c))
+    out[:A.shape[0], :A.shape[1]] = A
+    # [tile][output][chunk][term / 8][lane group][term % 2]
+    #   -> [tile][chunk][lane group][output][step = 2 (term / 8) + term % 2]
+    return np.ascontiguousarray(out.reshape(t, 16, c, 2, 4, 2).transpose(0, 2, 4, 1, 3, 5)).reshape(-1)
+
+
+def _chains(tab):
+    """Line tables [..., 4, M] as parity chains [..., even | odd, 4, 16 C], zero-padded;
+    C = 2, 4, 8 or 16 positions on each of 16 lanes."""
+    M = tab.shape[-1]
+    C = next(c for c in (2, 4, 8, 16) if 16 * c >= (M + 1) // 2)
+    out = tab.new_zeros(tab.shape[:-2] + (2, 4, 16 * C))
+    for q in (0, 1):
+        out[..., q, :, :(M + 1 - q) // 2] = tab[..., q::2]
+    return out
+
+
+def _halves(A, flip=0):
+    """The blocks of A that map modes of one parity to the even and to the odd
+    outputs (flip: from the opposite parity), packed alike."""
+    t, c = -(-((A.shape[0] + 1) // 2) // 16), -(-((A.shape[1] + 1) // 2) // 16)
+    return [pack_operator(A[q::2, (q + flip) % 2::2], t, c) for q in (0, 1)]
+
+
 class _SplitRhs:
     """Launch 7 with the right-hand-side product split along K: one launch of
     the partial products (batch over field x K slice), then
@@ -326,6 +378,8 @@ class Plan:
                 raise TypeError("launch %r cannot be recorded in a step plan" % launch.name)
         elif isinstance(launch, _Gemm):
             check(lib.pypde_plan_add_gemm(h, ctypes.byref(launch.desc)), launch.name)
+        elif isinstance(launch, _Phase):
+            check(lib.pypde_plan_add_phase(h, *launch.args), launch.name)
         elif isinstance(launch, _GemmGroup):
             if launch.split:
                 for m in launch.members:
@@ -518,6 +572,14 @@ class RBCBatch:
                 H = L1 // 2
                 ops_y = np.stack([ay.G[:H, 0::2], ay.G[:H, 1::2], ay.Gd[:H, 0::2], ay.Gd[:H, 1::2]])
                 self.yfold = dict(B=T(ops_y), sv=sv[0], sd=sd[0])
+        # the phases need the mirror symmetry of every transform operator
+        # (present on any Gauss-Lobatto grid) and lines that fit their blocks
+        most = 512   # PYPDE_STAGE_MAX_MODES
+        self.staged = (self.group_launches and not self.exact_solves
+                       and 6 <= min(M0, M1) and max(M0, M1) <= most and max(L0, L1) <= 2 * most
+                       and all(_mirror_signs(A, A.shape[0]) == [sg] for A, sg in
+                               ((ax.G, 1.0), (ax.Gd, -1.0), (ax.GT, 1.0), (ax.GdT, -1.0),
+                                (ay.G, 1.0), (ay.Gd, -1.0), (ax.BF.T, 1.0), (ay.BF.T, 1.0))))
         self.PBy = T(np.stack([ay.B, ay.BD]))                                 # [2, M1, N1]
         self.BSy = T(ay.BS)                                                   # [M1, M1]
         K = L0 + N0 + M0 + (2 * M0 if self.beta != 1.0 else 0)
@@ -612,10 +674,12 @@ class RBCBatch:
         if self.yfold is None and (self.nstage > 1 or self.beta != 1.0):
             raise NotImplementedError("RK3 and beta != 1 need even dealiased lengths in y "
                                       "(the y-folded layout)")
+        if self.staged:
+            self._stage_operators(ax, ay, pm, T)
         # candidate K splits of the right-hand-side product (few instances only)
         tiles = 3 * B * ((M0 + 31) // 32) * ((M1 + 31) // 32)
         self._splits = [S for S in (2, 3, 4, 6, 8) if L0 % S == 0 and L0 // S >= 32] \
-            if (tiles <= 768 and self.group_launches) else []
+            if (tiles <= 768 and self.group_launches and not self.staged) else []
         # every workspace of the step is a view into one buffer (the step plan's
         # workspace region); the K-split partials come last, so that a plan
         # that keeps fewer slices needs a shorter workspace
@@ -629,6 +693,13 @@ class RBCBatch:
             wsd += [("Y2", (B, 3, 2 * L0, 2 * L1)), ("Pr", (B, 3, L0, L1))]
         wsd += [("Z", (B, 3, L0, M1)), ("Rb", (B, 3, M0, M1)), ("div", (B, N0, N1)),
                 ("W2", (B, 2, M0, N1 + M1)), ("RP", (B, M0, M1)), ("W1", (B, M0, N1 + 2 * M1))]
+        if self.staged:
+            H1 = (L1 + 1) // 2
+            wsd = [("Y1", (B, 3, 2, L0, M1)), ("Pr", (B, 3, 2, L0, H1)), ("Z", (B, 3, L0, M1)),
+                   ("Rb", (B, 3, M0, M1)), ("W2", (B, 2, M0, M1)), ("W2v", (B, M0, N1)),
+                   ("RP", (B, M0, M1)), ("W1", (B, 2, M0, M1)), ("div", (B, N0, N1))]
+            if self.nstage > 1:   # the previous stage's velocities (c-term)
+                wsd.append(("uv", (B, 4, L0, H1)))
         if self._splits:
             wsd += [("rhs_work", (3 * B * max(self._splits), M0, M1))]
         offs, total = {}, 0
@@ -648,6 +719,61 @@ class RBCBatch:
         self.graph_steps = 0
         self.graphs = {}  # captured graphs by their number of steps
         self.plan = None
+
+    def _stage_operators(self, ax, ay, pm, T):
+        """The packed operators and tables of the phases (pypde_rbc_stage)."""
+        H0, H1 = (self.L0 + 1) // 2, (self.L1 + 1) // 2
+
+        def dev(parts):
+            return T(np.concatenate([np.asarray(p).reshape(-1) for p in parts]))
+
+        def half(A, H):   # even and odd terms of the first H outputs
+            t, c = -(-H // 16), -(-((A.shape[1] + 1) // 2) // 16)
+            return [pack_operator(A[:H, q::2], t, c) for q in (0, 1)]
+
+        def modal(A, H):  # even and odd outputs over the first H points
+            t, c = -(-((A.shape[0] + 1) // 2) // 16), -(-H // 16)
+            return [pack_operator(A[q::2, :H], t, c) for q in (0, 1)]
+        Q, Hy = pm["Qy"], pm["Hy"]
+        k0, k1 = np.arange(self.M0), np.arange(self.M1)
+        self.stage_ops = dict(
+            gx=dev(sum((half(A, H0) for A in (ax.G, ax.Gd, ax.GT, ax.GdT)), [])),
+            gy=dev(half(ay.G, H1) + half(ay.Gd, H1)),
+            bfy=dev(modal(ay.BF, H1)), bfx=dev(modal(ax.BF, H0)),
+            wy=dev([pack_operator(Hy @ ay.C), pack_operator(Hy @ ay.Cd), pack_operator(ay.Cd)]),
+            qy=dev([pack_operator(Q), pack_operator(ay.TSn @ Q), pack_operator(ay.TDSn @ Q)]),
+            cdx=dev(_halves(ax.Cd, 1)), corr=dev(_halves(ax.TDSn, 1) + _halves(ax.TSn)),
+            bds=dev([_diags(ax.B @ ax.Cd, (-1, 1, 3, 5)), _diags(ax.BS, (-2, 0, 2, 4))]),
+            sn=dev([-(k / (k + 2.0)) ** 2 for k in (k0, k1)]))
+        # [parity][LM | R | MU | NU][line][chain position]
+        self.stage_prec = _chains(self.precT.transpose(0, 1)).permute(1, 2, 0, 3).contiguous()
+
+    def _phase_launches(self, L, st):
+        """Stage `st` as eight launches (pypde_rbc_phase)."""
+        B, M0, M1, L0, L1 = self.B, self.M0, self.M1, self.L0, self.L1
+        tag = "" if self.nstage == 1 else "[%d]" % st
+        a, r = RbcStage(), self._rhs_args(st)
+        r.rows_per_thread = 1
+        ptrs = dict(X=self.X, pres=self.pres, P=self.P, Y1=self.Y1, Pr=self.Pr, Z=self.Z, R=self.Rb,
+                    W2=self.W2, W2v=self.W2v, RP=self.RP, W1=self.W1, div=self.div,
+                    uv=getattr(self, "uv", None), dtbc=self.dTbcdz1,
+                    hx=_chains(self.st_rhx[st]), hy=_chains(self.st_rhy[st]),
+                    prec=self.stage_prec, mdtb=self.st_mdtb[st],
+                    idta=self.st_idta[st], nu=self.t_nu, **self.stage_ops)
+        for n, t in ptrs.items():
+            setattr(a, n, t.data_ptr() if t is not None else None)
+        a.beta = self.beta
+        a.ratio = float(self.kc[st]) / float(self.kb[st])
+        a.N0, a.N1, a.M0, a.M1, a.L0, a.L1, a.batch = self.N0, self.N1, M0, M1, L0, L1, B
+        self._keep += [a, r, ptrs]
+        # operations of the products as run (halves; triangular operators from
+        # their first nonzero chunk on)
+        fl = (6 * L0 * M0 * M1, 8 * L0 * L1 * M1, 3 * L0 * L1 * M1, 3 * L0 * M0 * M1,
+              5 * M0 * M1 * M1, M0 * M0 * M1 // 2, 6 * M0 * M1 * M1, 2 * M0 * M0 * M1)
+        names = ("xpass+rhs_banded", "yproducts", "z_conv", "rhs+helmholtz_x", "helmholtz_y+div_y",
+                 "poisson_lines+div_x", "poisson_qy+corr_y", "correct+pres")
+        for i, name in enumerate(names):
+            L.append(_Phase(name + tag, a, r if i == 0 else None, i + 1, float(B) * fl[i]))
 
     def _helmholtz_matrix(self, st, b, f, axis):
         """Dense Helmholtz operator B S - lam I S of stage st, instance b, field
@@ -731,6 +857,9 @@ class RBCBatch:
         L = []
         for st in range(self.nstage):
             S = []
+            if self.staged:
+                self._phase_launches(L, st)
+                continue
             self._stage_launches(S, st)
             if self.group_launches:
                 _group_launches(S, "" if self.nstage == 1 else "[%d]" % st)
@@ -764,12 +893,7 @@ class RBCBatch:
             self._plain_y_launches(L, tag)
         # 5-6  banded part R_f of the right-hand side from the stage-start state:
         #      constant, pressure gradient, old value, buoyancy, explicit diffusion
-        a = RbcRhs()
-        a.X, a.pres, a.cst, a.R = p(X), p(self.pres), p(self.st_const[st]), p(self.Rb)
-        a.mdta, a.dta = p(self.st_mdta[st]), p(self.st_dta[st])
-        a.fdiff = p(self.st_fdiff[st]) if self.diffusion else None
-        a.tx, a.ty = p(self.tx), p(self.ty)
-        a.M0, a.M1, a.N0, a.N1, a.batch = M0, M1, N0, N1, B
+        a = self._rhs_args(st)
         self._keep.append(a)
         L.append(_Call("rhs_banded" + tag, lib.pypde_rbc_rhs_banded, ctypes.byref(a)))
         # 7  X_f = BF_x Z_f + R_f   (the forward transform along x of the
@@ -858,6 +982,17 @@ class RBCBatch:
                        iB=_bidx(s1=M0 * NW, d1=2, s2=M1, m2=2), D=p(X), ldd=M1,
                        iD=_bidx(s1=3 * sX, d1=2, s2=sX, m2=2), beta=1.0, alpha=-1.0,
                        C=p(X), ldc=M1, iC=_bidx(s1=3 * sX, d1=2, s2=sX, m2=2)))
+
+    def _rhs_args(self, st):
+        """Arguments of the banded right-hand side of stage st."""
+        p = lambda t: t.data_ptr()
+        a = RbcRhs()
+        a.X, a.pres, a.cst, a.R = p(self.X), p(self.pres), p(self.st_const[st]), p(self.Rb)
+        a.mdta, a.dta = p(self.st_mdta[st]), p(self.st_dta[st])
+        a.fdiff = p(self.st_fdiff[st]) if self.diffusion else None
+        a.tx, a.ty = p(self.tx), p(self.ty)
+        a.M0, a.M1, a.N0, a.N1, a.batch = self.M0, self.M1, self.N0, self.N1, self.B
+        return a
 
     def _yfold_launches(self, L, st, tag):
         """y-pass, products and y forward transform in the y-folded layout.  RK3
@@ -1020,7 +1155,7 @@ class RBCBatch:
         """Autotune the kernel variant of every GEMM launch of the step (the
         state is restored afterwards, so in-place launches can be timed)."""
         from . import autotune
-        if not autotune.enabled():
+        if not autotune.enabled() or self.staged:
             return
         saved = [t.clone() for t in (self.X, self.pres, self.P)]
         s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -1204,7 +1339,7 @@ class RBCBatch:
             self.step_eager()
 
     def gemm_flops(self):
-        return sum(l.flops for l in self.launches if isinstance(l, _Gemm))
+        return sum(l.flops for l in self.launches if isinstance(l, (_Gemm, _Phase)))
 
 
 def transfer_function(TL, TM, TR, x, k=0.01):
