@@ -710,7 +710,7 @@ __global__ void __launch_bounds__(256) banded_axis1_win_kernel(LineGeom g, BandS
 // load of a wave is 64 consecutive entries of a row shifted by one band
 // offset, so all accesses coalesce and the shifted copies hit in cache.  The
 // sum is band_row's, term for term.  NDT: the number of diagonals when it is
-// known at compile time (3), else kMaxDiag.  Every load is unconditional: a
+// known at compile time (3, 4), else kMaxDiag.  Every load is unconditional: a
 // term that does not exist for this output (its column outside the input)
 // reads a clamped column and is left out of the sum, so the loads are not
 // placed behind per-lane branches that would wait for each in turn.
@@ -804,6 +804,9 @@ static int launch_banded(LineGeom g, const BandSpec& bs, int hint, void* stream,
         } else if (bs.nd == 3) {
             if (u8) hipLaunchKernelGGL((banded_axis1_res_kernel<8, false, 3>), grid, dim3(256), 0, st, g, bs);
             else hipLaunchKernelGGL((banded_axis1_res_kernel<4, false, 3>), grid, dim3(256), 0, st, g, bs);
+        } else if (bs.nd == 4) {
+            if (u8) hipLaunchKernelGGL((banded_axis1_res_kernel<8, false, 4>), grid, dim3(256), 0, st, g, bs);
+            else hipLaunchKernelGGL((banded_axis1_res_kernel<4, false, 4>), grid, dim3(256), 0, st, g, bs);
         } else {
             if (u8) hipLaunchKernelGGL((banded_axis1_res_kernel<8, false, kMaxDiag>), grid, dim3(256), 0, st, g, bs);
             else hipLaunchKernelGGL((banded_axis1_res_kernel<4, false, kMaxDiag>), grid, dim3(256), 0, st, g, bs);
