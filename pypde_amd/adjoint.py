@@ -480,17 +480,20 @@ class Trajectory:
         self.e.pres.copy_(pres)
 
     def run(self, X0, pres0, nsteps):
-        """J_nu and the checkpoints; the engine state ends at step n."""
+        """J_nu and the checkpoints; the engine state ends at step n.  Nu is affine
+        in T, so its mean is that of the mean temperature: one addition per step
+        and one evaluation."""
         self._set(X0, pres0)
         cks = {0: self._state()}
-        acc = torch.zeros(self.e.B, dtype=ops.DTYPE, device=X0.device)
+        mean = torch.zeros_like(self.e.X[:, 2])
         ckpt = self._spacing(nsteps)
         for k in range(1, nsteps + 1):
             self._step()
-            acc += self.nu.value(self.e.X[:, 2])
+            mean += self.e.X[:, 2]
             if k % ckpt == 0 and k < nsteps:
                 cks[k] = self._state()
-        return acc / nsteps, cks
+        mean /= nsteps
+        return self.nu.value(mean), cks
 
     def grad_nusselt(self, X0, pres0, nsteps):
         """dJ_nu / d(X0, pres0) by the reverse sweep over checkpointed segments."""

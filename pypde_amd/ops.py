@@ -23,6 +23,9 @@ def device():
 def to_dev(a):
     """numpy / list / tensor -> contiguous float64 device tensor."""
     if isinstance(a, torch.Tensor):
+        if a.dtype is DTYPE and a.is_cuda and a.is_contiguous() and \
+                a.device.index == torch.cuda.current_device():
+            return a
         t = a.to(device=device(), dtype=DTYPE)
     else:
         arr = np.asarray(a, dtype=np.float64)
@@ -166,7 +169,9 @@ def _desc(ta, tb, m, n, k, batch, alpha, beta, A, lda, sA, B, ldb, sB, D, ldd, s
     d.A, d.B, d.C = A, B, C
     d.D = D
     d.lda, d.ldb, d.ldd, d.ldc = lda, ldb, ldd, ldc
-    d.iA, d.iB, d.iD, d.iC = _bi(sA), _bi(sB), _bi(sD), _bi(sC)
+    # plain strides: a fresh descriptor's other batch fields are zero, which the
+    # library reads as divisors of 1 and no moduli
+    d.iA.s1, d.iB.s1, d.iD.s1, d.iC.s1 = sA, sB, sD, sC
     d.alpha_vec = alpha_vec
     d.alpha_div = 1
     d.variant = 0
@@ -646,7 +651,7 @@ def recurrence_solve(tabs, x, axis=0, out=None, lpb=0, variant=None):
     if variant is None:
         from . import autotune
         key = ("rec", axis, n_in, n, g.nlines, g.batch, tabs.form(), tabs.per_line)
-        if autotune.enabled() and not autotune._capturing() and key not in autotune.cache():
+        if autotune.cached(key, None) is None and autotune.enabled() and not autotune._capturing():
             xs = _as3(x).clone()
             os_ = torch.empty(_out_shape(_as3(x), axis, n), dtype=DTYPE, device=x.device)
             gs = _geom(xs, os_, axis, n_in, n, lpb)
@@ -656,7 +661,7 @@ def recurrence_solve(tabs, x, axis=0, out=None, lpb=0, variant=None):
                 check(lib.pypde_recurrence_solve(ctypes.byref(gs), ctypes.byref(rs), s),
                       "pypde_recurrence_solve")
             autotune.choose(key, run, REC_CANDIDATES, default=0)
-        variant = autotune.cache().get(key, 0)
+        variant = autotune.cached(key, 0)
     r = tabs.struct(variant, lines)
     check(lib.pypde_recurrence_solve(ctypes.byref(g), ctypes.byref(r), s),
           "pypde_recurrence_solve")
