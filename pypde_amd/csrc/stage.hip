@@ -466,96 +466,112 @@ __global__ void __launch_bounds__(256) stage_zconv(Stage a, int ntask)
 }
 
 // ---------------------------------------------------------------------------
-// Phase 4: for 16 columns and the x modes of one parity, R += BF_x Z (the input
+// Phase 4: for 16 NT columns and the x modes of one parity, R += BF_x Z (the input
 // folded over the mirrored x rows while it is staged into LDS) and the Helmholtz
-// solve along x of those chains, in place on R.
-constexpr int kXsPitch = 24;  // 2 rows apart = 384 bytes: neighbouring lane groups read distinct banks
-
-template <int C>
-__global__ void __launch_bounds__(512) stage_rhs_hx(Stage a)
+// solve along x of those chains, in place on R.  One instance takes NT = 1 (96
+// blocks at 256 x 256) and everything early; batches NT = 2, which halves the
+// operator traffic from L2 (32 bytes per cycle and CU with 16 columns) and keeps two
+// blocks per CU: the right-hand side then reuses the LDS of the staged input and the
+// tables are read after the product.
+template <int C, int NT>
+__global__ void __launch_bounds__(512, NT == 1 ? 1 : 4) stage_rhs_hx(Stage a)
 {
     extern __shared__ double lds[];
+    // two rows apart = 128 bytes past a multiple of 256: neighbouring lane groups
+    // read distinct banks
+    constexpr int W = 16 * NT, XP = W + 8, YP = W + 1;
     const int M0 = a.M0, M1 = a.M1, L0 = a.L0, H0 = (L0 + 1) / 2;
-    const int kc = div_up(H0, 16), CT = div_up(M1, 16);
+    const int kc = div_up(H0, 16), CT = div_up(M1, W);
     double* Xs = lds;
-    double* Ys = lds + kc * 16 * kXsPitch;  // [16 C][17]
+    double* Ys = NT == 1 ? lds + kc * 16 * XP : lds;  // [16 C][YP]
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4, wave = tid >> 6;
     const int id = xcd_remap(blockIdx.x, gridDim.x);
-    const int q = id & 1, c0 = ((id >> 1) % CT) * 16, e = (id >> 1) / CT;
+    const int q = id & 1, c0 = ((id >> 1) % CT) * W, e = (id >> 1) / CT;
     const int rows = (M0 + 1 - q) / 2, RT = div_up((M0 + 1) / 2, 16);  // packed tiles of either parity
     const double* __restrict__ Z = a.Z + (long long)e * L0 * M1;
     double* __restrict__ R = a.R + (long long)e * M0 * M1;
+    const int tc = tid % W, tr = tid / W;
     {
-        const int col = min(c0 + (tid & 15), M1 - 1);
-        for (int k0 = tid >> 4; k0 < kc * 16; k0 += 8 * 32) {
+        constexpr int RP = 512 / W;  // rows per pass
+        const int col = min(c0 + tc, M1 - 1);
+        for (int k0 = tr; k0 < kc * 16; k0 += 8 * RP) {
             double u[8], d[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                const int k = min(k0 + 32 * s, H0 - 1);
+                const int k = min(k0 + RP * s, H0 - 1);
                 u[s] = Z[(long long)k * M1 + col];
                 d[s] = Z[(long long)(L0 - 1 - k) * M1 + col];
             }
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
-                const int k = k0 + 32 * s;
+                const int k = k0 + RP * s;
                 if (k >= kc * 16) break;
                 const double sum = k == L0 - 1 - k ? u[s] : (q ? u[s] - d[s] : u[s] + d[s]);
-                Xs[k * kXsPitch + (tid & 15)] = k < H0 ? sum : 0.0;
+                Xs[k * XP + tc] = k < H0 ? sum : 0.0;
             }
         }
     }
-    // tiles of this wave: wave, wave + 8 (at most 16 C / 16 = C tiles)
+    // tiles of this wave: wave, wave + 8 (at most C tiles)
     constexpr int TW = (C + 7) / 8;
-    double add[TW][4];
-    const int col = c0 + n;
+    double add[TW][NT][4];
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = (wave + 8 * t) * 16 + g + 4 * u;
+                add[t][j][u] = R[(long long)min(2 * i + q, M0 - 1) * M1 + min(c0 + 16 * j + n, M1 - 1)];
+            }
     double tab[4][C];   // of the chain this thread solves below
-    if (tid < 256) chain_tables<C>(tab, a.hx + ((long long)e * 2 + q) * 4 * 16 * C, 16 * C, tid & 15);
-#pragma unroll
-    for (int j = 0; j < TW; ++j)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int i = (wave + 8 * j) * 16 + g + 4 * u;
-            add[j][u] = R[(long long)min(2 * i + q, M0 - 1) * M1 + min(col, M1 - 1)];
-        }
+    const double* __restrict__ hx = a.hx + ((long long)e * 2 + q) * 4 * 16 * C;
+    if (NT == 1 && tid < 256) chain_tables<C>(tab, hx, 16 * C, tid & 15);
     __syncthreads();
     const double* __restrict__ op = a.bfx + (long long)q * RT * kc * kFrag;
+    v4d acc[TW][NT] = {};
 #pragma unroll
-    for (int j = 0; j < TW; ++j) {
-        const int t = wave + 8 * j;
-        if (t < RT) {
-            v4d acc = {};
-            v4d f[kDeep];
-            auto load = [&](int st, int k) { f[st] = op_frag(op, t, kc, k, lane); };
+    for (int t = 0; t < TW; ++t) {
+        if (wave + 8 * t < RT) {
+            constexpr int D = NT == 1 ? kDeep : 3;
+            v4d f[D];
+            auto load = [&](int st, int k) { f[st] = op_frag(op, wave + 8 * t, kc, k, lane); };
             auto compute = [&](int st, int k) {
 #pragma unroll
                 for (int s = 0; s < 4; ++s)
-                    acc = mfma(f[st][s], Xs[term(k, g, s) * kXsPitch + n], acc);
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[t][j] = mfma(f[st][s], Xs[term(k, g, s) * XP + 16 * j + n], acc[t][j]);
             };
-            pipeline<kDeep>(0, kc, load, compute);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int i = t * 16 + g + 4 * u;
-                Ys[i * 17 + n] = i < rows ? add[j][u] + acc[u] : 0.0;
-            }
-        } else if (t < C) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) Ys[(t * 16 + g + 4 * u) * 17 + n] = 0.0;
+            pipeline<D>(0, kc, load, compute);
         }
     }
+    if (NT > 1) {
+        chain_tables<C>(tab, hx, 16 * C, tid & 15);
+        __syncthreads();  // every wave is done with Xs
+    }
+#pragma unroll
+    for (int t = 0; t < TW; ++t)
+        if (wave + 8 * t < C)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int i = (wave + 8 * t) * 16 + g + 4 * u;
+                    Ys[i * YP + 16 * j + n] = i < rows ? add[t][j][u] + acc[t][j][u] : 0.0;
+                }
     __syncthreads();
-    if (tid < 256) {
+    if (tid < 256 * NT) {
         const int line = tid >> 4, c = tid & 15;
         double v[C];
 #pragma unroll
-        for (int k = 0; k < C; ++k) v[k] = Ys[(c * C + k) * 17 + line];
+        for (int k = 0; k < C; ++k) v[k] = Ys[(c * C + k) * YP + line];
         chain_solve<C>(v, tab, lane);
 #pragma unroll
-        for (int k = 0; k < C; ++k) Ys[(c * C + k) * 17 + line] = v[k];
+        for (int k = 0; k < C; ++k) Ys[(c * C + k) * YP + line] = v[k];
     }
     __syncthreads();
-    if (c0 + (tid & 15) < M1)
-        for (int i = tid >> 4; i < rows; i += 32)
-            R[(long long)(2 * i + q) * M1 + c0 + (tid & 15)] = Ys[i * 17 + (tid & 15)];
+    if (c0 + tc < M1)
+        for (int i = tr; i < rows; i += 512 / W) R[(long long)(2 * i + q) * M1 + c0 + tc] = Ys[i * YP + tc];
 }
 
 // ---------------------------------------------------------------------------
@@ -959,14 +975,24 @@ static void allow_lds(F fn, size_t bytes)
         (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+constexpr long long kRhsAlone = 700000;
+
 static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
 {
     pypde_rbc_rhs rhs{};
     unsigned nbr = 0;
     if (r) {
         rhs = *r;
-        const long long tr = (3LL * rhs.M0 * rhs.M1 * rhs.batch + 255) / 256;
-        nbr = (unsigned)std::min<long long>(tr, 16384);
+        const long long outs = 3LL * rhs.M0 * rhs.M1 * rhs.batch;
+        if (outs >= kRhsAlone) {
+            // many outputs: the tile form shares each row's y sums in LDS and runs
+            // by itself (64 x 256^2: 219 us; one output per thread 311)
+            rhs.rows_per_thread = 16;
+            const int rc = pypde_rbc_rhs_banded(&rhs, s);
+            if (rc != OK) return rc;
+        } else {
+            nbr = (unsigned)std::min<long long>((outs + 255) / 256, 16384);
+        }
     }
     const int HT = up((a.L0 + 1) / 2, 16);
     // 2 x 2 tiles per wave (half the operand traffic) once they give every
@@ -974,6 +1000,9 @@ static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
     const long long big = 3LL * a.batch * up(a.M1, 32) * 2 * up(HT, 2);
     if (big >= 2048) {
         hipLaunchKernelGGL((stage_xpass<2, 2, 2>), dim3(nbr + blocks4(big)), dim3(256), 0, s, a, rhs, nbr, (int)big);
+    } else if (3LL * a.batch * up(a.M1, 16) * 2 * up(HT, 2) >= 2048) {
+        const long long t = 3LL * a.batch * up(a.M1, 16) * 2 * up(HT, 2);
+        hipLaunchKernelGGL((stage_xpass<2, 1, 2>), dim3(nbr + blocks4(t)), dim3(256), 0, s, a, rhs, nbr, (int)t);
     } else {
         const long long t = 3LL * a.batch * up(a.M1, 16) * 2 * HT;
         hipLaunchKernelGGL((stage_xpass<1, 1, 4>), dim3(nbr + blocks4(t)), dim3(256), 0, s, a, rhs, nbr, (int)t);
@@ -1001,14 +1030,25 @@ static int phase3(const Stage& a, hipStream_t s)
     return check_launch("pypde_rbc_phase 3");
 }
 
+template <int C, int NT>
+static int phase4_n(const Stage& a, hipStream_t s)
+{
+    const size_t x = (size_t)up((a.L0 + 1) / 2, 16) * 16 * (16 * NT + 8), y = (size_t)16 * C * (16 * NT + 1);
+    const size_t lds = (NT == 1 ? x + y : std::max(x, y)) * sizeof(double);
+    allow_lds(stage_rhs_hx<C, NT>, lds);
+    const long long blocks = 2LL * 3 * a.batch * up(a.M1, 16 * NT);
+    hipLaunchKernelGGL((stage_rhs_hx<C, NT>), dim3((unsigned)blocks), dim3(512), lds, s, a);
+    return check_launch("pypde_rbc_phase 4");
+}
+
 template <int C>
 static int phase4_c(const Stage& a, hipStream_t s)
 {
-    const size_t lds = ((size_t)up((a.L0 + 1) / 2, 16) * 16 * kXsPitch + 16 * C * 17) * sizeof(double);
-    allow_lds(stage_rhs_hx<C>, lds);
-    const long long blocks = 2LL * 3 * a.batch * up(a.M1, 16);
-    hipLaunchKernelGGL(stage_rhs_hx<C>, dim3((unsigned)blocks), dim3(512), lds, s, a);
-    return check_launch("pypde_rbc_phase 4");
+    // 32 columns per block once that still gives every CU two blocks (64 x 256^2: 152
+    // us against 226); the longest chains would spill registers in that form
+    if constexpr (C < 16)
+        if (6LL * a.batch * up(a.M1, 32) >= 512) return phase4_n<C, 2>(a, s);
+    return phase4_n<C, 1>(a, s);
 }
 
 template <int C>
@@ -1018,10 +1058,11 @@ static int phase5_c(const Stage& a, hipStream_t s)
     const int len = 16 * kc;
     const size_t lds = 16 * (size_t)((len + 2 * (len / (2 * C))) | 1) * sizeof(double);
     allow_lds(stage_hy<C>, lds);
-    // four operator tiles per block until that fills the device, else more, so
-    // that the solve is repeated less often
+    // four operator tiles per block while the blocks run side by side (two per CU,
+    // one with the longest chains), else more, so that the solve is repeated less
+    // often (512 x 512: 800 blocks of four tiles 60 us)
     int per = 4;
-    while (per < 16 && (long long)rows * (up(kc, per) + up(kc + TN, per)) > 1024) per *= 2;
+    while (per < 16 && (long long)rows * (up(kc, per) + up(kc + TN, per) + 1) > (C == 16 ? 256 : 512)) per *= 2;
     const int p0 = up(kc, per), p1 = up(kc + TN, per);
     hipLaunchKernelGGL(stage_hy<C>, dim3((unsigned)(rows * (p0 + p1 + 1))), dim3(512), lds, s, a, p0, p1, per);
     return check_launch("pypde_rbc_phase 5");
