@@ -907,13 +907,19 @@ extern "C" int pypde_cheb_deriv(const pypde_lines* in, const double* s, int orde
     PYPDE_REQUIRE(g.len_out == n, "derivative output length must be %d", n);
     PYPDE_REQUIRE(n >= 3 || order == 0, "derivative needs n >= 3");
     if (g.nlines == 0 || g.batch == 0) return OK;
-    // lines per block: as many as 64 KB of LDS hold (or the hint), at most 16
+    // the lengths and hints of the line solves: a panel of whole lines beside its
+    // stencil within 64 KB
+    const int ntab = s ? g.len_in : 0;
+    const long long wl = pick_lines_per_block(g.pitch, ntab, in->lines_per_block, g.nlines);
+    PYPDE_REQUIRE((wl * g.pitch + ntab) * 8 <= kLdsBudget, "pypde_cheb_deriv: line length %d too long for an LDS panel",
+                  g.pitch);
+    // lines per block: as many as 64 KB of LDS hold (or the hint), at most 16; one
+    // line of the greatest length takes up to 120 bytes more with the entries that a
+    // chain may read below it
     const int cap = in->lines_per_block > 0 ? in->lines_per_block : 16;
     auto fits = [&](int w, size_t bytes) { return w <= cap && (w == 1 || w / 2 < g.nlines) && bytes <= (size_t)kLdsBudget; };
     g.W = fits(16, deriv_lds<16>(g.axis, n)) ? 16 : fits(8, deriv_lds<8>(g.axis, n)) ? 8
         : fits(4, deriv_lds<4>(g.axis, n)) ? 4 : fits(2, deriv_lds<2>(g.axis, n)) ? 2 : 1;
-    PYPDE_REQUIRE(g.W > 1 || deriv_lds<1>(g.axis, n) <= (size_t)kLdsBudget + 2 * kDerivU * sizeof(double),
-                  "pypde_cheb_deriv: line length %d too long for an LDS panel", n);
     const long long blocks = (long long)((g.nlines + g.W - 1) / g.W) * g.batch;
     PYPDE_REQUIRE(blocks < (1LL << 31), "pypde_cheb_deriv: grid too large");
     const DerivArgs a{g, s, order, scale_pow};

@@ -135,6 +135,29 @@ def test_engine_launch_records_without_gpu():
     assert b"regions" in lib.pypde_last_error()
 
 
+def test_derivative_line_lengths_without_gpu():
+    """pypde_cheb_deriv takes the line lengths and block hints that the line
+    solves take, and refuses the rest before anything is launched: 8191 entries,
+    with the stencil 4095, and hints whose panel fits."""
+    from pypde_amd import _lib
+    lib = _lib.lib
+
+    def refused(len_in, stencil, hint=0):
+        g = _lib.Lines()
+        g.src = g.dst = 1 << 20
+        g.len_in, g.len_out = len_in, len_in + (2 if stencil else 0)
+        g.nlines, g.lines_per_block = 100, hint
+        g.batch = 2 ** 31 - 1   # beyond any grid, which is checked after the lengths
+        assert lib.pypde_cheb_deriv(ctypes.byref(g), 1 << 21 if stencil else None, 1, 1.0,
+                                    None) != 0
+        msg = lib.pypde_last_error()
+        assert b"too long" in msg or b"grid" in msg, msg
+        return b"too long" in msg
+    assert not refused(8191, False) and refused(8192, False)
+    assert not refused(4095, True) and refused(4096, True) and refused(8190, True)
+    assert not refused(1000, False, hint=8) and refused(1000, False, hint=16)
+
+
 def test_multi_launch_packing_without_gpu():
     """The multi launches' host packing (no kernel runs): member ranges, the
     work total and the argument checks."""
