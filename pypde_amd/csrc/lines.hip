@@ -389,7 +389,8 @@ __device__ __forceinline__ void deriv_chain(double* x, int n, int p)
     const int jl = p ? 1 : 2;                 // last output of the chain (d_0 follows)
     const int nwin = ((n - 2) / 2 + kDerivU) / kDerivU;  // windows, the same for every lane
     const double c1 = x[P];
-    double acc = 0.0, cur[kDerivU], nxt[kDerivU];
+    // d_{n-2} is its product alone (-0 + y is y for every y), d_{n-3} follows d_{n-1} = 0
+    double acc = top ? 0.0 : -0.0, cur[kDerivU], nxt[kDerivU];
     double* q = x + jt * P;
 #pragma unroll
     for (int u = 0; u < kDerivU; ++u) cur[u] = q[(1 - 2 * u) * P];

@@ -140,6 +140,24 @@ def test_derivative_panels_bit_exact(amd, axis, N, lines, batch):
             assert np.array_equal(d, ref), (key, k)
 
 
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("N", [3, 4, 5, 18, 33])
+def test_derivative_signed_zeros(amd, axis, N):
+    """Zeros keep the recurrence's sign: the entry below the last is a product
+    alone, so a negative zero stays one, and the entries after it add to that."""
+    pypde_amd, ops, torch = amd
+    from oracle import pypde_oracle as o
+    b, ob = pypde_amd.Base(N, "CH"), o.Basis(N, "CH")
+    rng = np.random.default_rng(N)
+    v = np.full((N, 9), -0.0)
+    v[:, 3:] = rng.choice([-0.0, 0.0, 1.0, -1.0], size=(N, 6))
+    v = v if axis == 0 else np.ascontiguousarray(v.T)
+    for k in (1, 2):
+        d = host(b.derivative(ops.to_dev(v), k, axis=axis))
+        ref = o._along(lambda a: ob.derivative(a, k), v, axis)
+        assert np.array_equal(d, ref) and np.array_equal(np.signbit(d), np.signbit(ref)), k
+
+
 @pytest.mark.parametrize("N", [16, 64, 256])
 @pytest.mark.parametrize("axis", [0, 1])
 def test_fdma_bit_exact_and_transpose(amd, N, axis):
