@@ -359,7 +359,7 @@ struct StencilInvOp {
 // the even and the odd outputs, in the reference's order of additions (the
 // results are bit-identical).  What bounds one field of a few hundred points is
 // latency: the block's loads, one chain of n / 2 steps, the stores.  So a block
-// takes few lines (W <= 16: a 128 x 128 field is 8 blocks), the products
+// takes few lines (W = 16: a 128 x 128 field is 8 blocks), the products
 // 2 (j+1) c_{j+1} and the division by scale_pow are spread over all threads with
 // eight loads in flight, and a chain step is one LDS read, one addition and one
 // LDS write at offsets known at compile time.  A lane reads its next inputs
@@ -414,8 +414,8 @@ __device__ __forceinline__ void deriv_chain(double* x, int n, int p)
     wave_lds_sync();
 }
 
-template <int AXIS, int W>
-__global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
+template <int AXIS, int W, int NT>
+__global__ void __launch_bounds__(NT) cheb_deriv_kernel(DerivArgs a)
 {
     // along rows an odd pitch: neighbouring entries of a line in other banks
     constexpr int P = AXIS == 0 ? W : (W | 1);
@@ -430,7 +430,7 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
     const double* __restrict__ src = g.src + (long long)b * g.src_bs;
     double* __restrict__ dst = g.dst + (long long)b * g.dst_bs;
     const int tid = threadIdx.x;
-    // elements e = tid + 256 q of the panel: (k, c) with c fastest along columns
+    // elements e = tid + NT q of the panel: (k, c) with c fastest along columns
     // (the last panel's missing columns are clamped and not stored), k fastest
     // along rows
     const int total = AXIS == 0 ? n * W : n * nl;
@@ -438,12 +438,12 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
         if (AXIS == 0) { k = e / W; c = e % W; }
         else { c = e / n; k = e - c * n; }
     };
-    for (int e0 = tid; e0 < total; e0 += 256 * kDerivU) {
+    for (int e0 = tid; e0 < total; e0 += NT * kDerivU) {
         double v[kDerivU], v2[kDerivU];
 #pragma unroll
         for (int u = 0; u < kDerivU; ++u) {
             int k, c;
-            split(min(e0 + 256 * u, total - 1), k, c);
+            split(min(e0 + NT * u, total - 1), k, c);
             c = min(c, nl - 1);
             const long long at = AXIS == 0 ? l0 + c : (long long)(l0 + c) * g.src_ld;
             const long long st = AXIS == 0 ? g.src_ld : 1;
@@ -452,9 +452,9 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
         }
 #pragma unroll
         for (int u = 0; u < kDerivU; ++u) {
-            if (e0 + 256 * u >= total) break;
+            if (e0 + NT * u >= total) break;
             int k, c;
-            split(e0 + 256 * u, k, c);
+            split(e0 + NT * u, k, c);
             double y = v[u];
             if (a.s && k >= 2) {
                 const double tt = a.s[k - 2] * v2[u];
@@ -467,19 +467,20 @@ __global__ void __launch_bounds__(256) cheb_deriv_kernel(DerivArgs a)
     for (int o = 0; o < a.order; ++o) {
         __syncthreads();
         if (o > 0) {
-            for (int e = tid; e < n * W; e += 256) {
+            for (int e = tid; e < n * W; e += NT) {
                 const int k = e / W, c = e % W;
                 if (k >= 2) lds[k * P + c] = (double)(2 * k) * lds[k * P + c];
             }
             __syncthreads();
         }
-        // a lane pair per line: W even lanes, then W odd lanes (lanes past the
-        // last line repeat it)
+        // a lane pair per line, all in one wave: W even lanes, then W odd lanes
+        // (lanes past the last line repeat it)
+        static_assert(2 * W <= kWave, "both lanes of a line run in step");
         if (tid < 2 * W) deriv_chain<P>(lds + min(tid % W, nl - 1), n, tid / W);
     }
     __syncthreads();
     const double sp = a.scale_pow;
-    for (int e = tid; e < total; e += 256) {
+    for (int e = tid; e < total; e += NT) {
         int k, c;
         split(e, k, c);
         if (c >= nl) continue;
@@ -495,12 +496,20 @@ static size_t deriv_lds(int axis, int n)
     return (size_t)(n + 2 * kDerivU) * (axis == 0 ? W : (W | 1)) * sizeof(double);
 }
 
-template <int W>
-static void launch_deriv(const DerivArgs& a, unsigned blocks, hipStream_t s)
+template <int W, int NT>
+static int launch_deriv_nt(const DerivArgs& a, unsigned blocks, hipStream_t s)
 {
     const size_t shmem = deriv_lds<W>(a.g.axis, a.g.len_out);
-    if (a.g.axis == 0) hipLaunchKernelGGL((cheb_deriv_kernel<0, W>), dim3(blocks), dim3(256), shmem, s, a);
-    else hipLaunchKernelGGL((cheb_deriv_kernel<1, W>), dim3(blocks), dim3(256), shmem, s, a);
+    if (a.g.axis == 0) hipLaunchKernelGGL((cheb_deriv_kernel<0, W, NT>), dim3(blocks), dim3(NT), shmem, s, a);
+    else hipLaunchKernelGGL((cheb_deriv_kernel<1, W, NT>), dim3(blocks), dim3(NT), shmem, s, a);
+    return check_launch("pypde_cheb_deriv");
+}
+
+template <int W>
+static int launch_deriv(const DerivArgs& a, unsigned blocks, int threads, hipStream_t s)
+{
+    return threads == 64 ? launch_deriv_nt<W, 64>(a, blocks, s)
+         : threads == 128 ? launch_deriv_nt<W, 128>(a, blocks, s) : launch_deriv_nt<W, 256>(a, blocks, s);
 }
 
 // Upper two-band back substitution (twodma.f90:2-25).
@@ -921,17 +930,28 @@ extern "C" int pypde_cheb_deriv(const pypde_lines* in, const double* s, int orde
     auto fits = [&](int w, size_t bytes) { return w <= cap && (w == 1 || w / 2 < g.nlines) && bytes <= (size_t)kLdsBudget; };
     g.W = fits(16, deriv_lds<16>(g.axis, n)) ? 16 : fits(8, deriv_lds<8>(g.axis, n)) ? 8
         : fits(4, deriv_lds<4>(g.axis, n)) ? 4 : fits(2, deriv_lds<2>(g.axis, n)) ? 2 : 1;
+    // More panels than the device holds at a time: throughput counts, so a short
+    // panel takes 32 lines and as many threads as have 8 to 12 of its entries each
+    // (columns, 400,000 lines, first order: length 8 45 us with 16 lines and 256
+    // threads, 13 with 32 and 64; length 32 64 and 33; 64 96 and 94).  Fewer panels
+    // are bound by latency: all threads.
+    int threads = 256;
+    if (in->lines_per_block <= 0 && (long long)((g.nlines + g.W - 1) / g.W) * g.batch > 1024) {
+        if (g.W == 16 && g.nlines > 16 && n <= 48) g.W = 32;
+        threads = n * g.W <= 512 ? 64 : n * g.W <= 1536 ? 128 : 256;
+    }
     const long long blocks = (long long)((g.nlines + g.W - 1) / g.W) * g.batch;
     PYPDE_REQUIRE(blocks < (1LL << 31), "pypde_cheb_deriv: grid too large");
     const DerivArgs a{g, s, order, scale_pow};
+    const unsigned nb = (unsigned)blocks;
     switch (g.W) {
-    case 16: launch_deriv<16>(a, (unsigned)blocks, as_stream(stream)); break;
-    case 8: launch_deriv<8>(a, (unsigned)blocks, as_stream(stream)); break;
-    case 4: launch_deriv<4>(a, (unsigned)blocks, as_stream(stream)); break;
-    case 2: launch_deriv<2>(a, (unsigned)blocks, as_stream(stream)); break;
-    default: launch_deriv<1>(a, (unsigned)blocks, as_stream(stream)); break;
+    case 32: return launch_deriv<32>(a, nb, threads, as_stream(stream));
+    case 16: return launch_deriv<16>(a, nb, threads, as_stream(stream));
+    case 8: return launch_deriv<8>(a, nb, threads, as_stream(stream));
+    case 4: return launch_deriv<4>(a, nb, threads, as_stream(stream));
+    case 2: return launch_deriv<2>(a, nb, threads, as_stream(stream));
+    default: return launch_deriv<1>(a, nb, threads, as_stream(stream));
     }
-    return check_launch("pypde_cheb_deriv");
 }
 
 static int fdma_common(const pypde_lines* in, const double* l, const double* d, const double* u1,

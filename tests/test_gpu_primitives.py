@@ -141,6 +141,29 @@ def test_derivative_panels_bit_exact(amd, axis, N, lines, batch):
 
 
 @pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("N,lines,batch", [(3, 33000, 1), (16, 40, 700), (17, 33, 520), (20, 3, 1100), (48, 36, 400),
+                                           (49, 16, 1030), (97, 17, 600), (31, 1, 1025)])
+def test_derivative_many_short_lines_bit_exact(amd, axis, N, lines, batch):
+    """The derivative over more than 1024 panels, where short lines take 32 to a
+    panel and 64 or 128 threads: lengths on both sides of each choice, partial
+    panels, both orders, with and without the stencil, bit for bit the oracle's."""
+    pypde_amd, ops, torch = amd
+    from oracle import pypde_oracle as o
+    rng = np.random.default_rng(N)
+    for key in ("CH", "CD") if N > 4 else ("CH",):
+        b, ob = pypde_amd.Base(N, key), o.Basis(N, key)
+        M = N if key == "CH" else N - 2
+        v = rng.standard_normal((M, batch * lines))
+        x = v.reshape(M, batch, lines).transpose(1, 0, 2) if axis == 0 else v.T.reshape(batch, lines, M)
+        for k in (1, 2):
+            d = host(b.derivative(ops.to_dev(np.ascontiguousarray(x)), k, axis=axis, scale_pow=0.3))
+            ref = ob.derivative(v, k) / 0.3
+            ref = ref.reshape(N, batch, lines).transpose(1, 0, 2) if axis == 0 else \
+                ref.T.reshape(batch, lines, N)
+            assert np.array_equal(d, ref), (key, k)
+
+
+@pytest.mark.parametrize("axis", [0, 1])
 @pytest.mark.parametrize("N", [3, 4, 5, 18, 33])
 def test_derivative_signed_zeros(amd, axis, N):
     """Zeros keep the recurrence's sign: the entry below the last is a product
