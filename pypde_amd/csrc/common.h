@@ -1,8 +1,10 @@
 // Shared helpers for the pypde_amd HIP library (gfx950, wave64).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include <cstdio>
 #include <cstdarg>
+#include <mutex>
 #include <string>
 
 namespace pypde {
@@ -78,3 +80,28 @@ long long products_multi_bytes();
             return ::pypde::ERR_HIP;                                           \
         }                                                                      \
     } while (0)
+
+namespace pypde {
+
+// Asks for `bytes` of dynamic LDS for a kernel, whose static LDS counts towards the
+// default limit too: once per kernel, device and larger size, before its launch.
+// The limit is only ever raised.
+template <auto Kernel>
+int allow_lds(size_t bytes)
+{
+    constexpr int kDevices = 64;
+    static std::atomic<size_t> granted[kDevices];
+    static std::mutex raising;
+    int dev = 0;
+    PYPDE_HIP(hipGetDevice(&dev));
+    PYPDE_REQUIRE(dev >= 0 && dev < kDevices, "device %d not in 0..%d", dev, kDevices - 1);
+    if (granted[dev].load(std::memory_order_acquire) >= bytes) return OK;
+    std::lock_guard<std::mutex> lock(raising);
+    if (granted[dev].load(std::memory_order_relaxed) >= bytes) return OK;
+    PYPDE_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    granted[dev].store(bytes, std::memory_order_release);
+    return OK;
+}
+
+}  // namespace pypde

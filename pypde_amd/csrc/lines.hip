@@ -500,7 +500,10 @@ template <int W, int NT>
 static int launch_deriv_nt(const DerivArgs& a, unsigned blocks, hipStream_t s)
 {
     const size_t shmem = deriv_lds<W>(a.g.axis, a.g.len_out);
-    if (a.g.axis == 0) hipLaunchKernelGGL((cheb_deriv_kernel<0, W, NT>), dim3(blocks), dim3(NT), shmem, s, a);
+    const bool cols = a.g.axis == 0;
+    if (const int rc = cols ? allow_lds<cheb_deriv_kernel<0, W, NT>>(shmem) : allow_lds<cheb_deriv_kernel<1, W, NT>>(shmem))
+        return rc;
+    if (cols) hipLaunchKernelGGL((cheb_deriv_kernel<0, W, NT>), dim3(blocks), dim3(NT), shmem, s, a);
     else hipLaunchKernelGGL((cheb_deriv_kernel<1, W, NT>), dim3(blocks), dim3(NT), shmem, s, a);
     return check_launch("pypde_cheb_deriv");
 }

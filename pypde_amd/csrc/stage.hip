@@ -967,14 +967,6 @@ static int chain_len(int m)
     return c <= 2 ? 2 : c <= 4 ? 4 : c <= 8 ? 8 : 16;
 }
 
-// More than 64 KB of dynamic LDS has to be asked for, once per kernel.
-template <class F>
-static void allow_lds(F fn, size_t bytes)
-{
-    if (bytes > 64 * 1024)
-        (void)hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
 constexpr long long kRhsAlone = 700000;
 
 static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
@@ -1035,7 +1027,7 @@ static int phase4_n(const Stage& a, hipStream_t s)
 {
     const size_t x = (size_t)up((a.L0 + 1) / 2, 16) * 16 * (16 * NT + 8), y = (size_t)16 * C * (16 * NT + 1);
     const size_t lds = (NT == 1 ? x + y : std::max(x, y)) * sizeof(double);
-    allow_lds(stage_rhs_hx<C, NT>, lds);
+    if (const int rc = allow_lds<stage_rhs_hx<C, NT>>(lds)) return rc;
     const long long blocks = 2LL * 3 * a.batch * up(a.M1, 16 * NT);
     hipLaunchKernelGGL((stage_rhs_hx<C, NT>), dim3((unsigned)blocks), dim3(512), lds, s, a);
     return check_launch("pypde_rbc_phase 4");
@@ -1057,7 +1049,7 @@ static int phase5_c(const Stage& a, hipStream_t s)
     const int kc = up(a.M1, 16), TN = up(a.N1, 16), rows = a.batch * up(a.M0, 16);
     const int len = 16 * kc;
     const size_t lds = 16 * (size_t)((len + 2 * (len / (2 * C))) | 1) * sizeof(double);
-    allow_lds(stage_hy<C>, lds);
+    if (const int rc = allow_lds<stage_hy<C>>(lds)) return rc;
     // four operator tiles per block while the blocks run side by side (two per CU,
     // one with the longest chains), else more, so that the solve is repeated less
     // often (512 x 512: 800 blocks of four tiles 60 us)
@@ -1074,7 +1066,7 @@ static int phase6_c(const Stage& a, hipStream_t s)
     const unsigned nbp = 2u * a.batch * up(a.M1, 16);
     const long long t = 2LL * a.batch * up((a.N0 + 1) / 2, 16) * up(a.N1, 16);
     const size_t lds = (16 * C * 17 + 2 * (16 * C + 4) * 16 + 8 * 16 * C) * sizeof(double);
-    allow_lds(stage_poisson<C>, lds);
+    if (const int rc = allow_lds<stage_poisson<C>>(lds)) return rc;
     hipLaunchKernelGGL(stage_poisson<C>, dim3(nbp + blocks4(t)), dim3(256), lds, s, a, nbp, (int)t);
     return check_launch("pypde_rbc_phase 6");
 }

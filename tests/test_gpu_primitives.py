@@ -164,6 +164,17 @@ def test_derivative_many_short_lines_bit_exact(amd, axis, N, lines, batch):
 
 
 @pytest.mark.parametrize("axis", [0, 1])
+def test_derivative_longest_lines_bit_exact(amd, axis):
+    """Lines of 8191 entries, whose one-line panel takes a little more than 64 KB
+    of LDS."""
+    pypde_amd, ops, torch = amd
+    from oracle import pypde_oracle as o
+    v = np.random.default_rng(8191).standard_normal((8191, 3))
+    d = host(ops.cheb_deriv(ops.to_dev(v if axis == 0 else np.ascontiguousarray(v.T)), axis))
+    assert np.array_equal(d if axis == 0 else d.T, o.diff_2d(v))
+
+
+@pytest.mark.parametrize("axis", [0, 1])
 @pytest.mark.parametrize("N", [3, 4, 5, 18, 33])
 def test_derivative_signed_zeros(amd, axis, N):
     """Zeros keep the recurrence's sign: the entry below the last is a product
