@@ -542,44 +542,45 @@ class RBCBatch:
                                np.vstack([ax.GT, ax.GdT])]))                   # [3, 2L0, M0]
         self.GGy = T(np.vstack([ay.G, ay.Gd]))                                # [2L1, M1]
         self.BFy = T(ay.BF)                                                   # [M1, L1]
-        # parity-folded halves of the transform operators (even lengths only)
+        # signs of the transform operators' mirror symmetry (present on any
+        # Gauss-Lobatto grid; BF[i, L-1-j] = s (-1)^i BF[i, j])
+        sg = {n: _mirror_signs(A, A.shape[0]) for n, A in
+              (("Gx", ax.G), ("Gdx", ax.Gd), ("GTx", ax.GT), ("GdTx", ax.GdT), ("Gy", ay.G),
+               ("Gdy", ay.Gd), ("BFx", ax.BF.T), ("BFy", ay.BF.T))}
+        sg = {n: s[0] if s is not None else None for n, s in sg.items()}
+        # the phases need that symmetry of every operator and lines that fit their blocks
+        most = 512   # PYPDE_STAGE_MAX_MODES
+        self.staged = (self.group_launches and not self.exact_solves
+                       and 6 <= min(M0, M1) and max(M0, M1) <= most and max(L0, L1) <= 2 * most
+                       and all(s == (-1.0 if n in ("Gdx", "GdTx", "Gdy") else 1.0)
+                               for n, s in sg.items()))
+        # parity-folded halves of the transform operators (even lengths only) for
+        # the step with one launch per operator
         self.fold_x = self.fold_y = self.fold_bf = None
-        if M0 % 2 == 0 and L0 % 2 == 0:
-            GG = [np.vstack([ax.G, ax.Gd]), np.vstack([ax.GT, ax.GdT])]
-            sg = [_mirror_signs(g, L0) for g in GG]
-            if sg[0] is not None and sg[0] == sg[1]:
-                tops = [np.vstack([g[:L0 // 2], g[L0:L0 + L0 // 2]]) for g in (GG[0], GG[0], GG[1])]
-                self.fold_x = dict(E=T(np.stack([t[:, 0::2] for t in tops])),
-                                   O=T(np.stack([t[:, 1::2] for t in tops])), sign=_sign_bits(sg[0]))
-        if M1 % 2 == 0 and L1 % 2 == 0:
-            GGy_h = np.vstack([ay.G, ay.Gd])
-            sg = _mirror_signs(GGy_h, L1)
-            if sg is not None:
-                top = np.vstack([GGy_h[:L1 // 2], GGy_h[L1:L1 + L1 // 2]])
-                self.fold_y = dict(E=T(top[:, 0::2]), O=T(top[:, 1::2]), sign=_sign_bits(sg))
-            sg = _mirror_signs(ay.BF.T, L1)   # BF[i, L1-1-j] = s (-1)^i BF[i, j]
-            if sg is not None:
-                h = L1 // 2
-                self.fold_bf = dict(B=T(np.stack([ay.BF[0::2, :h], ay.BF[1::2, :h]])), sign=sg[0])
+        sx = [sg["Gx"], sg["Gdx"]]
+        if M0 % 2 == 0 and L0 % 2 == 0 and not self.staged and None not in sx \
+                and sx == [sg["GTx"], sg["GdTx"]]:
+            tops = [np.vstack([g[:L0 // 2], d[:L0 // 2]])
+                    for g, d in ((ax.G, ax.Gd), (ax.G, ax.Gd), (ax.GT, ax.GdT))]
+            self.fold_x = dict(E=T(np.stack([t[:, 0::2] for t in tops])),
+                               O=T(np.stack([t[:, 1::2] for t in tops])), sign=_sign_bits(sx))
+        sy = [sg["Gy"], sg["Gdy"]]
+        even_y = M1 % 2 == 0 and L1 % 2 == 0
+        H = L1 // 2
+        if even_y and not self.staged and None not in sy:
+            top = np.vstack([ay.G[:H], ay.Gd[:H]])
+            self.fold_y = dict(E=T(top[:, 0::2]), O=T(top[:, 1::2]), sign=_sign_bits(sy))
+        if even_y and not self.staged and sg["BFy"] is not None:
+            self.fold_bf = dict(B=T(np.stack([ay.BF[0::2, :H], ay.BF[1::2, :H]])), sign=sg["BFy"])
         # y-folded layout of the dealiased fields: the y-pass writes even / odd
         # coefficient halves over the first half of the y grid and the products
         # kernel reconstructs both mirrored columns (half-size plain GEMMs)
         self.yfold = None
-        if self.fold_y is not None and self.fold_bf is not None:
-            sv = _mirror_signs(ay.G, L1)
-            sd = _mirror_signs(ay.Gd, L1)
-            if sv is not None and sd is not None:
-                H = L1 // 2
-                ops_y = np.stack([ay.G[:H, 0::2], ay.G[:H, 1::2], ay.Gd[:H, 0::2], ay.Gd[:H, 1::2]])
-                self.yfold = dict(B=T(ops_y), sv=sv[0], sd=sd[0])
-        # the phases need the mirror symmetry of every transform operator
-        # (present on any Gauss-Lobatto grid) and lines that fit their blocks
-        most = 512   # PYPDE_STAGE_MAX_MODES
-        self.staged = (self.group_launches and not self.exact_solves
-                       and 6 <= min(M0, M1) and max(M0, M1) <= most and max(L0, L1) <= 2 * most
-                       and all(_mirror_signs(A, A.shape[0]) == [sg] for A, sg in
-                               ((ax.G, 1.0), (ax.Gd, -1.0), (ax.GT, 1.0), (ax.GdT, -1.0),
-                                (ay.G, 1.0), (ay.Gd, -1.0), (ax.BF.T, 1.0), (ay.BF.T, 1.0))))
+        if even_y and None not in sy and sg["BFy"] is not None:
+            self.yfold = dict(sv=sy[0], sd=sy[1])
+            if not self.staged:
+                self.yfold["B"] = T(np.stack([ay.G[:H, 0::2], ay.G[:H, 1::2],
+                                              ay.Gd[:H, 0::2], ay.Gd[:H, 1::2]]))
         self.PBy = T(np.stack([ay.B, ay.BD]))                                 # [2, M1, N1]
         self.BSy = T(ay.BS)                                                   # [M1, M1]
         K = L0 + N0 + M0 + (2 * M0 if self.beta != 1.0 else 0)
@@ -599,7 +600,8 @@ class RBCBatch:
         self.BSTx = T(ax.BST)                                                 # [M0, M0]
         # the forward step applies the banded blocks as diagonals
         # (pypde_rbc_rhs_banded) and only the forward transform BF densely
-        self.BFx = T(ax.BF)                                                   # [M0, L0]
+        if not self.staged:
+            self.BFx = T(ax.BF)                                               # [M0, L0]
         self.tx = T(np.vstack([_diags(ax.BD, (1, 3, 5)), _diags(ax.B, (0, 2, 4)),
                                _diags(ax.BS, (-2, 0, 2, 4)), _diags(ax.BST, (-2, 0, 2, 4)),
                                _diags(ax.BD2S, (0, 2)), _diags(ax.BD2ST, (0, 2))]))   # [18, M0]
@@ -622,13 +624,15 @@ class RBCBatch:
         #   RP = B_x div H_y^T = (B [Cd | C])_x [X_f (H_y C_f)^T]_f
         #   W1 = P W_y^T = RP (W_y Q_y)^T, row 0 with row 0 of Q_y zeroed (the
         #        gauge P[0,0] = 0 of the solve)
-        self.HCy = T(np.stack([np.vstack([ay.C, pm["Hy"] @ ay.C]),
-                               np.vstack([ay.Cd, pm["Hy"] @ ay.Cd])]))        # [2, N1+M1, M1]
-        self.BCx = T(ax.B @ np.hstack([ax.Cd, ax.C]))                         # [M0, 2M0]
-        Qy0 = np.array(pm["Qy"], copy=True)
-        Qy0[0, :] = 0.0
-        self.WQy = T(Wy @ pm["Qy"])                                           # [N1+2M1, M1]
-        self.WQy0 = T(Wy @ Qy0)
+        #   (the phases hold their own packed forms)
+        if not self.staged:
+            self.HCy = T(np.stack([np.vstack([ay.C, pm["Hy"] @ ay.C]),
+                                   np.vstack([ay.Cd, pm["Hy"] @ ay.Cd])]))    # [2, N1+M1, M1]
+            self.BCx = T(ax.B @ np.hstack([ax.Cd, ax.C]))                     # [M0, 2M0]
+            Qy0 = np.array(pm["Qy"], copy=True)
+            Qy0[0, :] = 0.0
+            self.WQy = T(Wy @ pm["Qy"])                                       # [N1+2M1, M1]
+            self.WQy0 = T(Wy @ Qy0)
         self.Snx = T(ax.Sn)                                                   # [N0, M0]
         self.Acorr = T(np.stack([ax.TDSn, ax.TSn]))                           # [2, M0, M0]
 

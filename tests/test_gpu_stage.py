@@ -22,6 +22,9 @@ def _run(shape, B, case, integrator, beta):
     for group in (True, False):
         e = RBCBatch(shape, params, case=case, integrator=integrator, beta=beta, group_launches=group)
         assert e.staged == group and (len(e.launches) == 8 * e.nstage) == group
+        # neither form sets up the other's operators
+        assert hasattr(e, "stage_ops") == group
+        assert not group or not (e.fold_x or e.fold_y or e.fold_bf or hasattr(e, "WQy"))
         if group:
             k0, k1 = np.arange(e.N0), np.arange(e.N1)
             fall = np.exp(-8.0 * k0 / e.N0)[:, None] * np.exp(-8.0 * k1 / e.N1)
