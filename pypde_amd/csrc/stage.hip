@@ -51,6 +51,7 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double v2u __attribute__((ext_vector_type(2), aligned(8)));  // pair at any 8-byte address
 typedef double v2a __attribute__((ext_vector_type(2)));
 
+constexpr int kCus = 256;   // of the device
 constexpr int kFrag = 256;  // doubles per operator fragment (16 outputs x 16 terms)
 
 // term of chunk k that lane group g takes at step s
@@ -263,26 +264,26 @@ __global__ void __launch_bounds__(256) stage_xpass(Stage a, pypde_rbc_rhs r, uns
 
 // ---------------------------------------------------------------------------
 // Phase 2: the eight dealiased fields (u, v, and both derivatives of u, v, T) at
-// 16 x-rows and 32 mirrored pairs of y points, one field per wave, and the
+// 16 x-rows and 16 NY mirrored pairs of y points, one field per wave, and the
 // convective products of rbc_products (pointwise.hip), folded for the forward
 // transform: Pr[e][sum | difference][L0][H1].  The fields never reach memory;
 // with the c-term (ratio != 0) the previous stage's velocities come from uv and
 // this stage's go there ([b][u | v][point | mirror][L0][H1], each entry read and
 // written by one thread).
 constexpr int kYPitch = 34;  // a wave's 16 x 32 tile of its rows: the rows' pairs in distinct banks
-constexpr int kNY = 2;       // tiles of 16 point pairs per block
 
+template <int NY>  // tiles of 16 point pairs per block
 __global__ void __launch_bounds__(512) stage_yprod(Stage a)
 {
     __shared__ union {
         double x[8][16 * kYPitch];
-        double field[8][2][kNY][16][17];
+        double field[8][2][NY][16][17];
     } sh;
     auto& buf = sh.field;
     const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int M1 = a.M1, L0 = a.L0, L1 = a.L1, H1 = (L1 + 1) / 2;
-    const int HT = div_up(H1, 16), YG = div_up(HT, kNY), RG = div_up(L0, 16);
+    const int HT = div_up(H1, 16), YG = div_up(HT, NY), RG = div_up(L0, 16);
     const int kc = div_up((M1 + 1) / 2, 16);
     const int id = xcd_remap(blockIdx.x, gridDim.x);
     const int yg = id % YG, rr = id / YG;
@@ -294,8 +295,8 @@ __global__ void __launch_bounds__(512) stage_yprod(Stage a)
     const double* __restrict__ op = a.gy + (long long)dy * 2 * HT * kc * kFrag;  // [q][HT][kc]
     double* xs = sh.x[wave];
     {
-        v4d acc[2][kNY] = {};
-        v4d f[2][2][kNY];
+        v4d acc[2][NY] = {};
+        v4d f[2][2][NY];
         v2u x[2][4];
         auto load = [&](int st, int k) {
             // rows g, g + 4, ..., 16 lanes along each
@@ -305,8 +306,8 @@ __global__ void __launch_bounds__(512) stage_yprod(Stage a)
 #pragma unroll
             for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int j = 0; j < kNY; ++j)
-                    f[st][q][j] = op_frag(op, q * HT + min(yg * kNY + j, HT - 1), kc, k, lane);
+                for (int j = 0; j < NY; ++j)
+                    f[st][q][j] = op_frag(op, q * HT + min(yg * NY + j, HT - 1), kc, k, lane);
         };
         auto compute = [&](int st, int k) {
             wave_lds_sync();  // the previous chunk is read
@@ -319,7 +320,7 @@ __global__ void __launch_bounds__(512) stage_yprod(Stage a)
                 const v2a p = *reinterpret_cast<const v2a*>(xs + n * kYPitch + 2 * term(0, g, s));
                 const double ev = pair_first(p, 2 * term(k, g, s), M1);
 #pragma unroll
-                for (int j = 0; j < kNY; ++j) {
+                for (int j = 0; j < NY; ++j) {
                     acc[0][j] = mfma(ev, f[st][0][j][s], acc[0][j]);
                     acc[1][j] = mfma(p.y, f[st][1][j][s], acc[1][j]);
                 }
@@ -330,7 +331,7 @@ __global__ void __launch_bounds__(512) stage_yprod(Stage a)
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int j = 0; j < kNY; ++j)
+            for (int j = 0; j < NY; ++j)
 #pragma unroll
                 for (int u = 0; u < 4; ++u) buf[wave][q][j][g + 4 * u][n] = acc[q][j][u];
     }
@@ -339,8 +340,8 @@ __global__ void __launch_bounds__(512) stage_yprod(Stage a)
     {
 #pragma clang fp contract(off)
         const int j = t >> 8, ri = (t >> 4) & 15, ln = t & 15;
-        const int i = r0 + ri, l = (yg * kNY + j) * 16 + ln;
-        if (i >= L0 || l >= H1) return;
+        const int i = r0 + ri, l = (yg * NY + j) * 16 + ln;
+        if (j >= NY || i >= L0 || l >= H1) return;
         double E[8], O[8];
 #pragma unroll
         for (int w = 0; w < 8; ++w) {
@@ -1004,8 +1005,12 @@ static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
 
 static int phase2(const Stage& a, hipStream_t s)
 {
-    const int HT = up((a.L1 + 1) / 2, 16);
-    hipLaunchKernelGGL(stage_yprod, dim3((unsigned)(a.batch * up(a.L0, 16) * up(HT, kNY))), dim3(512), 0, s, a);
+    const int HT = up((a.L1 + 1) / 2, 16), rows = a.batch * up(a.L0, 16);
+    // two tiles per block halve the traffic of the rows; while single tiles find a CU
+    // each, they are done in two thirds of the time (224 x 224: 9.4 us against 13.3,
+    // 16 x 300: 10.7 against 16.4; 240 x 240 with 276 blocks: 15.4 against 14.8)
+    if (rows * HT <= kCus) hipLaunchKernelGGL(stage_yprod<1>, dim3((unsigned)(rows * HT)), dim3(512), 0, s, a);
+    else hipLaunchKernelGGL(stage_yprod<2>, dim3((unsigned)(rows * up(HT, 2))), dim3(512), 0, s, a);
     return check_launch("pypde_rbc_phase 2");
 }
 

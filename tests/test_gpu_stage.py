@@ -46,6 +46,7 @@ def _run(shape, B, case, integrator, beta):
 @pytest.mark.parametrize("shape,B", [((8, 8), 1), ((9, 11), 2), ((34, 35), 1), ((36, 66), 2), ((67, 33), 1),
                                      ((66, 98), 1), ((130, 21), 1), ((20, 131), 2), ((259, 18), 1),
                                      ((16, 258), 1), ((514, 12), 1), ((12, 513), 1), ((12, 460), 1),
+                                     ((240, 224), 1), ((240, 240), 1), ((12, 260), 3),
                                      ((130, 131), 64)])
 def test_phases_match_single_launches(shape, B):
     _run(shape, B, "rbc", "eu", 1.0)
