@@ -372,7 +372,8 @@ int pypde_rbc_rhs_banded(const pypde_rbc_rhs* args, void* stream);
  *
  * Operators are packed for the FP64 MFMA: op[tile][chunk][64][4], lane l and step s
  * holding A[16 tile + l % 16][16 chunk + 8 (s / 2) + 2 (l / 16) + s % 2], zero past A's
- * ends, where A's rows are outputs and its columns terms (of one mode parity where noted):
+ * ends, where A's rows are outputs and its columns terms (of one mode parity where noted).
+ * They must be 32-byte aligned; every other array 8-byte aligned, as any double:
  *   gx   [U,V | T][value | d/dx][even | odd modes] of the first H0 x points
  *   gy   [value | d/dy][even | odd modes] of the first H1 y points
  *   bfy, bfx  [even | odd output modes] over the first H1, H0 points

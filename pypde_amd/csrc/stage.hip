@@ -41,6 +41,7 @@
 #include "../../include/pypde_amd.h"
 
 #include <algorithm>
+#include <cstdint>
 
 namespace pypde {
 
@@ -1124,6 +1125,9 @@ extern "C" int pypde_rbc_phase(const pypde_rbc_stage* st, const pypde_rbc_rhs* r
                       a.gx && a.gy && a.bfy && a.bfx && a.wy && a.qy && a.cdx && a.corr && a.bds && a.sn &&
                       a.dtbc && a.hx && a.hy && a.prec && a.mdtb && a.idta && a.nu,
                   "null stage pointer");
+    for (const double* op : {a.gx, a.gy, a.bfy, a.bfx, a.wy, a.qy, a.cdx, a.corr})
+        PYPDE_REQUIRE(reinterpret_cast<uintptr_t>(op) % sizeof(v4d) == 0,
+                      "stage: packed operators are read 32 bytes at a time and must be 32-byte aligned");
     PYPDE_REQUIRE(a.ratio == 0.0 || a.uv, "the c-term needs the previous stage's velocities");
     PYPDE_REQUIRE((long long)a.batch * (a.L0 / 16 + 1) * (a.L1 / 16 + 1) * 6 < (1LL << 30), "stage: batch too large");
     if (rhs) {

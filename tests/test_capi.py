@@ -158,6 +158,35 @@ def test_derivative_line_lengths_without_gpu():
     assert not refused(1000, False, hint=8) and refused(1000, False, hint=16)
 
 
+def test_phase_arguments_without_gpu():
+    """pypde_rbc_phase checks its stage before anything runs: the packed
+    operators' alignment, the phase number, the geometry and its limits."""
+    from pypde_amd import _lib
+    lib = _lib.lib
+
+    def stage(**kw):
+        a = _lib.RbcStage()
+        for name, t in a._fields_:
+            if t is ctypes.c_void_p:
+                setattr(a, name, 1 << 20)
+        a.N0, a.N1, a.M0, a.M1, a.L0, a.L1, a.batch = 20, 16, 18, 14, 30, 24, 0
+        for k, v in kw.items():
+            setattr(a, k, v)
+        return a
+
+    def run(phase=1, **kw):
+        return lib.pypde_rbc_phase(ctypes.byref(stage(**kw)), None, phase, None)
+    assert run() == 0   # an empty batch: every check passes, nothing is launched
+    for op in ("gx", "gy", "bfy", "bfx", "wy", "qy", "cdx", "corr"):
+        assert run(**{op: (1 << 20) + 8}) != 0, op
+        assert b"aligned" in lib.pypde_last_error()
+    assert run(X=(1 << 20) + 8, prec=(1 << 20) + 8) == 0
+    assert run(phase=9) != 0 and b"phase" in lib.pypde_last_error()
+    assert run(M0=513, N0=515, L0=772) != 0 and b"modes" in lib.pypde_last_error()
+    assert run(qy=None) != 0 and b"null" in lib.pypde_last_error()
+    assert run(uv=None) == 0 and run(uv=None, ratio=-0.5) != 0
+
+
 def test_multi_launch_packing_without_gpu():
     """The multi launches' host packing (no kernel runs): member ranges, the
     work total and the argument checks."""
