@@ -17,9 +17,7 @@ between device synchronisations, replayed from HIP graphs of ten steps
 Also reported on the same line:
   roofline       the dominant launch of the timed step (largest time per step in an
                  eager pass of the same K steps with HIP events around each launch),
-                 timed as 20 back-to-back launches replayed from a HIP graph; for the
-                 K-split right-hand side, its GEMM kernel (partial products and the
-                 buoyancy product in one launch)
+                 timed as 20 back-to-back launches replayed from a HIP graph
   batched        64 instances of 256x256 (Ra log-uniform in [1e4, 1e7]) in one
                  batched step: aggregate instance-steps/s and the ratio to the plain path
   variants       the same 256x256 step with RK3 (three stages) and with beta = 0.5
@@ -61,26 +59,21 @@ def seeded_noise(shape, seed=0, amplitude=1e-3):
     return rng.uniform(-amplitude, amplitude, size=shape)
 
 
-# HBM bytes per launch of each launch of the 256x256 step (kernel choices of
-# pypde_amd/tune_db.json), from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE passes
-# over `python3 bench.py --steps 20 --warmup 2 --no-cpu --no-extra
-# --all-launches` (the mean over 20 graph-replayed launches of each), each
-# counter divided by what it reads for a device copy of known size
+# HBM bytes per launch of each phase of the 256x256 step, from rocprofv3 --pmc
+# FETCH_SIZE and WRITE_SIZE passes over `python3 bench.py --steps 20 --warmup 2
+# --no-cpu --no-extra --all-launches` (the mean over 20 graph-replayed launches of
+# each), each counter divided by what it reads for a device copy of known size
 # (`python3 bench.py --copy-calibration`); profiles/hbm_traffic_pmc.md gives the
 # commands, the calibration and the per-launch table.
 TRAFFIC_BYTES = {
-    "xpass": 12615994,
-    "ypass_v+ypass_x": 23615960,
-    "products+rhs_banded": 27793527,
-    "z_conv": 10696155,
-    "rhs": 13369201,
-    "helmholtz_x": 3658500,
-    "helmholtz_y": 3514573,
-    "div_y": 11533202,
-    "div_x+poisson_rhs": 12059385,
-    "poisson_lines": 3499907,
-    "poisson_qy+corr_y+corr_y0": 15145603,
-    "pres_p+correct": 10773292,
+    "xpass+rhs_banded": 26422872,
+    "yproducts": 15793951,
+    "z_conv": 9129285,
+    "rhs+helmholtz_x": 9543043,
+    "helmholtz_y+div_y": 15855639,
+    "poisson_lines+div_x": 7673231,
+    "poisson_qy+corr_y": 14733260,
+    "correct+pres": 8496136,
 }
 
 
@@ -122,9 +115,36 @@ def copy_calibration(mib=256, reps=5):
                                            "launches": reps, "kernel": "torch.mul(x, 1.0, out=y)"}}))
 
 
+def phase_bytes(phase, eng):
+    """Bytes that a phase of the step cannot do without: its fields read and
+    written once per instance, its operators and tables once."""
+    B, N0, N1, M0, M1, L0, L1 = eng.B, eng.N0, eng.N1, eng.M0, eng.M1, eng.L0, eng.L1
+    H0, H1, f = (L0 + 1) // 2, (L1 + 1) // 2, M0 * M1
+    fields, tables = {
+        # X, pres and the constant terms to Y1 and R
+        1: (3 * f + N0 * N1 + 3 * f + 6 * L0 * M1 + 3 * f, 4 * H0 * M0),
+        2: (6 * L0 * M1 + 6 * L0 * H1, 2 * H1 * M1 + L0 * L1),
+        3: (6 * L0 * H1 + 3 * L0 * M1, M1 * H1),
+        4: (3 * L0 * M1 + 2 * 3 * f, M0 * H0),
+        5: (3 * f + 3 * f + 2 * f + M0 * N1, (2 * M1 + N1) * M1),
+        # W2, V's divergence factor and U to RP and the divergence
+        6: (2 * f + M0 * N1 + f + f + N0 * N1, N0 * M0 // 2 + 4 * f),
+        7: (f + 3 * f, 3 * M1 * M1),
+        # W1, U, V, P, the divergence and the pressure; U, V and the pressure written
+        8: (2 * f + 2 * f + f + 2 * N0 * N1 + 2 * f + N0 * N1, M0 * M0),
+    }[phase]
+    return 8.0 * (B * fields + tables)
+
+
 def launch_cost(name, launch, eng):
-    """(bound, algorithmic amount per launch) of one launch of the fused step."""
-    from pypde_amd.engine import _Gemm, _GemmGroup
+    """(bound, algorithmic amount per launch) of one launch of the fused step; a
+    phase, which does both, by the one that takes longer at the device's peaks."""
+    from pypde_amd.engine import _Gemm, _GemmGroup, _Phase
+    if isinstance(launch, _Phase):
+        nbytes = phase_bytes(launch.args[2], eng)
+        if launch.flops / (FP64_PEAK_TFLOPS * 1e12) >= nbytes / (HBM_PEAK_GBS * 1e9):
+            return "mfma", launch.flops
+        return "hbm", nbytes
     if isinstance(launch, (_Gemm, _GemmGroup)):
         return "mfma", launch.flops
     B, N0, N1, M0, M1, L0, L1 = eng.B, eng.N0, eng.N1, eng.M0, eng.M1, eng.L0, eng.L1
@@ -625,17 +645,20 @@ def gemm_k_sweep(m=384, n=192, batch=18, ks=(16, 32, 64, 127, 254, 508), variant
 
 def gemm_variants():
     """Every plain GEMM kernel variant on each plain GEMM launch of the 256x256
-    step (single descriptors and grouped launches; the folded x-pass is not a
-    plain GEMM), timed like the tuner does; for the y-pass also with its A
-    operand read contiguously (ska = 1: the same shape without the
-    every-other-column access).  The engine state is restored afterwards."""
+    step with one launch per operator, the form with exact line solves (single
+    descriptors and grouped launches; the folded x-pass is not a plain GEMM, and
+    the phases of the default step have no variants), timed like the tuner does;
+    for the y-pass also with its A operand read contiguously (ska = 1: the same
+    shape without the every-other-column access).  The engine state is restored
+    afterwards."""
     import ctypes
     import torch
     from pypde_amd import autotune
     from pypde_amd._lib import GemmDesc, check, lib
     from pypde_amd.engine import _Gemm, _GemmGroup, _SplitRhs
     from pypde_amd.navier import NavierStokes
-    ns = NavierStokes(case="rbc", shape=(256, 256), ra=1e8, pr=1.0, dt=1e-3, tsave=None)
+    ns = NavierStokes(case="rbc", shape=(256, 256), ra=1e8, pr=1.0, dt=1e-3, tsave=None,
+                      exact_solves=True)
     eng = ns.engine
     eng.step_eager()
     torch.cuda.synchronize()
@@ -656,7 +679,7 @@ def gemm_variants():
     out = {}
     for l in eng.launches:
         for p in ([l.group] if isinstance(l, _SplitRhs) else [l]):
-            if isinstance(p, _GemmGroup) and p.members:
+            if isinstance(p, _GemmGroup):
                 descs = [GemmDesc.from_buffer_copy(m.desc) for m in p.members]
             elif isinstance(p, _Gemm) and p.desc.fold == 0:
                 descs = [GemmDesc.from_buffer_copy(p.desc)]
@@ -895,7 +918,8 @@ def main():
     ap.add_argument("--cpu-steps", type=int, default=150)
     ap.add_argument("--micro", action="store_true", help="run the microbench only")
     ap.add_argument("--gemm-variants", action="store_true",
-                    help="time every plain GEMM variant on the 256x256 step's GEMM launches")
+                    help="time every plain GEMM variant on the GEMM launches of the 256x256 step "
+                         "with one launch per operator")
     ap.add_argument("--gemm-k-sweep", action="store_true",
                     help="time a y-pass-shaped GEMM against K (fixed cost and cost per K slab)")
     ap.add_argument("--batched-launches", action="store_true",

@@ -1,17 +1,21 @@
 """Fused RBC2D time step on the GPU: a batch of same-shape instances with
 per-instance Rayleigh / Prandtl numbers and time steps.
 
-The Euler IMEX step of navier/rbc2d.py:396-434 is regrouped into eight kernel
-launches per stage whatever the batch size (RBCBatch._phase_launches, csrc/stage.hip):
+The Euler IMEX step of navier/rbc2d.py:396-434 is regrouped into eight phases per
+stage, one kernel launch each whatever the batch size but for the first, whose
+banded right-hand side has its own launch when it is large
+(RBCBatch._phase_launches, csrc/stage.hip):
 every separable 1-D operator chain of the reference (stencil -> derivative ->
 zero-pad -> DCT, forward DCT -> truncate -> pseudo-inverse B, ...) is folded into
 one dense operator per axis, applied on the FP64 matrix cores by parity or mirror
 halves; the Helmholtz and Poisson solves stay banded line solves with the
 reference's LU factors, in the launches of the products next to them.
 
-The step with one launch per operator (below, 17 or so launches) remains for
-exact_solves, for more modes per axis than a phase's lines hold, and as the
-member launches of a heterogeneous batch (group_launches=False).
+The step with one launch per operator (below, 17 or so launches; with
+group_launches some of them share one) remains for exact_solves, which also takes
+more than the 512 modes per axis that a phase's lines and the register recurrences
+hold, for fewer than 6 modes on an axis, and as the member launches of a
+persistent heterogeneous batch (group_launches=False).
 
 Data layout in HBM (float64, row-major):
   X    [B, 3, M0, M1]      Galerkin coefficients of U, V (ChebDirichlet^2) and
@@ -237,18 +241,14 @@ class _GemmGroup:
               self.name)
 
 
-class _Phase(_GemmGroup):
+class _Phase:
     """One phase of a stage (pypde_rbc_phase): the phase's independent products
     and line solves in one launch.  Its tiling follows from the sizes alone."""
 
     def __init__(self, name, stage, rhs, phase, flops):
-        self.name, self.flops, self.members, self.split = name, flops, [], False
+        self.name, self.flops = name, flops
         self.fn = lib.pypde_rbc_phase
         self.args = (ctypes.byref(stage), ctypes.byref(rhs) if rhs is not None else None, phase)
-
-    @property
-    def variant(self):
-        return self.args[2]
 
     def __call__(self, stream):
         check(self.fn(*self.args, stream), self.name)
@@ -360,8 +360,8 @@ class Plan:
         self.handle = h
 
     def add(self, launch):
-        """Record one launch (a _Gemm, _GemmGroup, _RecCall, _Call, _SplitRhs or
-        an ops.Recorded)."""
+        """Record one launch (a _Gemm, _GemmGroup, _RecCall, _Call, _SplitRhs,
+        _Phase or an ops.Recorded)."""
         h = self.handle
         if isinstance(launch, _SplitRhs):
             self.add(launch.group)
@@ -1298,7 +1298,8 @@ class RBCBatch:
     def variants(self):
         """{launch name: kernel variant} chosen for this step (GEMM variants;
         grouped launches: their variant or "split"; recurrences: 1 block form,
-        2 lane-chunk form, 3 block form with 32 lines per block)."""
+        2 lane-chunk form, 3 block form with 32 lines per block).  Phases have no
+        variants to choose: their forms follow from the sizes."""
         out = {l.name: l.desc.variant for l in self.launches if isinstance(l, _Gemm)}
         out.update({l.name: ("split" if l.split else l.variant) for l in self.launches
                     if isinstance(l, _GemmGroup)})

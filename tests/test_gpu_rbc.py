@@ -84,12 +84,14 @@ def test_multi_step_graph_matches_single_steps(golden):
 
 def test_grouped_launches_match_separate(golden):
     """The step with independent GEMMs sharing launches equals the step with
-    one launch per GEMM (kernel variants may differ: 1e-13)."""
+    one launch per GEMM (kernel variants may differ: 1e-13).  Engines with exact
+    line solves: the others of this size run the step in phases."""
     import torch
     from pypde_amd.engine import RBCBatch, _GemmGroup, _SplitRhs
     pre = "step_rbc_eu_in_"
-    engs = [RBCBatch((20, 16), [dict(ra=1e5, pr=1.0, dt=0.01)], case="rbc", group_launches=g)
-            for g in (True, False)]
+    engs = [RBCBatch((20, 16), [dict(ra=1e5, pr=1.0, dt=0.01)], case="rbc", group_launches=g,
+                     exact_solves=True) for g in (True, False)]
+    assert not any(e.staged for e in engs)
     assert any(isinstance(l, (_GemmGroup, _SplitRhs)) for l in engs[0].launches)
     assert not any(isinstance(l, (_GemmGroup, _SplitRhs)) for l in engs[1].launches)
     for e in engs:
@@ -102,6 +104,41 @@ def test_grouped_launches_match_separate(golden):
     for t in ("X", "pres"):
         a, b = (host(getattr(e, t)) for e in engs)
         assert rel(a, b) < 1e-13, t
+
+
+@pytest.mark.parametrize("integrator", ["eu", "rk3"])
+def test_grouped_and_split_launches_in_a_plan(integrator):
+    """Grouped launches and the right-hand-side product split along K, run one by
+    one and as recorded in the step plan: bit for bit the same, and the step with
+    one launch per GEMM within 1e-12 (the product's sum in another order, which
+    the line solves amplify)."""
+    import torch
+    from pypde_amd.engine import RBCBatch, _GemmGroup, _SplitRhs
+    shape, params = (48, 40), [dict(ra=1e5, pr=1.0, dt=5e-3), dict(ra=1e6, pr=0.7, dt=2e-3)]
+    engs = [RBCBatch(shape, params, case="rbc", integrator=integrator, group_launches=g,
+                     exact_solves=True) for g in (True, False)]
+    for rhs, cands in engs[0]._rhs_pairs:
+        for i, l in enumerate(engs[0].launches):
+            if l is rhs or any(l is c for c in cands.values()):
+                engs[0].launches[i] = cands[2]
+    kinds = [type(l) for l in engs[0].launches]
+    assert kinds.count(_SplitRhs) == engs[0].nstage and _GemmGroup in kinds
+    rng = np.random.default_rng(2)
+    fall = np.exp(-8.0 * np.arange(48) / 48)[:, None] * np.exp(-8.0 * np.arange(40) / 40)
+    X = torch.as_tensor(0.05 * rng.standard_normal((2, 3, 46, 38)) * fall[:46, :38])
+    pres = torch.as_tensor(0.01 * rng.standard_normal((2, 48, 40)) * fall)
+    out = []
+    for e, step in ((engs[0], engs[0].step_launches), (engs[0], engs[0].step_eager),
+                    (engs[1], engs[1].step_eager)):
+        e.X.copy_(X)
+        e.pres.copy_(pres)
+        e.P.zero_()
+        step()
+        out.append([host(t).copy() for t in (e.X, e.pres, e.P)])
+    for one, plan in zip(out[0], out[1]):
+        assert np.array_equal(one, plan)
+    for i in (0, 1):
+        assert rel(out[1][i], out[2][i]) < 1e-12, i
 
 
 @pytest.mark.parametrize("case", ["linear", "rbc"])
