@@ -351,9 +351,10 @@ typedef struct pypde_rbc_rhs {
 
 int pypde_rbc_rhs_banded(const pypde_rbc_rhs* args, void* stream);
 
-/* One stage of the fused step in eight launches (pypde_rbc_phase), each a set of
- * independent blocks that hold whole lines of one axis; the phases of a stage run
- * in order on one stream.  State and workspace are row-major per instance b and
+/* One stage of the fused step in eight phases (pypde_rbc_phase), each a set of
+ * independent blocks that hold whole lines of one axis, in one launch (the first in
+ * two when its right-hand side is large); the phases of a stage run in order on one
+ * stream.  State and workspace are row-major per instance b and
  * field f; E = 3 b + f.  H0, H1 = (L0 + 1) / 2, (L1 + 1) / 2.
  *   1  Y1[E][value | d/dx][L0][M1] from X; with rhs also R (pypde_rbc_rhs_banded)
  *   2  Pr[E][sum | difference over the mirrored y points][L0][H1], the convective
@@ -398,7 +399,9 @@ typedef struct pypde_rbc_stage {
     int N0, N1, M0, M1, L0, L1, batch;
 } pypde_rbc_stage;
 
-/* phase 1..8; rhs only with phase 1 (or NULL; rows_per_thread must be 1) */
+/* phase 1..8; rhs only with phase 1 (or NULL).  rows_per_thread must be 1: the phase
+ * picks the form, one output per thread in its own launch or, from 700,000 outputs
+ * (3 M0 M1 batch) on, the tile form in a launch before it; the values are the same. */
 int pypde_rbc_phase(const pypde_rbc_stage* stage, const pypde_rbc_rhs* rhs, int phase, void* stream);
 
 /* pypde_rbc_products_yfold and pypde_rbc_rhs_banded (one output per thread:

@@ -3,8 +3,8 @@ resolutions, Rayleigh / Prandtl numbers and time steps, advanced together by
 one HIP-graph launch per step (or per `nsteps` steps).
 
 Instances are grouped by shape into size classes; each class is an
-`engine.RBCBatch` (one launch per operator for all its instances, GEMM and
-banded schedules autotuned for that shape).  The captured graph forks one
+`engine.RBCBatch` (the step's phases for all its instances; in the persistent
+form one launch per operator, whose GEMM and banded schedules are autotuned).  The captured graph forks one
 stream branch per size class from the capture stream and joins them at the
 end of every step, so classes of small fields overlap on the device instead of
 running one after another.  No reference counterpart: the reference steps one

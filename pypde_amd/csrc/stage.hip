@@ -1,4 +1,5 @@
-// One stage of the fused RBC2D step (navier/rbc2d.py:396-434) in eight launches.
+// One stage of the fused RBC2D step (navier/rbc2d.py:396-434) in eight phases, a launch
+// each (the first takes two when its right-hand side is large).
 //
 // The dense operators of the step act on one axis at a time, and every banded
 // solve runs along one axis, so the work falls into phases that each need whole
@@ -969,7 +970,16 @@ static int chain_len(int m)
     return c <= 2 ? 2 : c <= 4 ? 4 : c <= 8 ? 8 : 16;
 }
 
+// Outputs from which the right-hand side leaves the x-pass's launch for one of its
+// own, whose tiles share each row's y sums in LDS.  Below, a launch costs more than
+// they save.  Phase 1 merged against alone: 256 x 256 (194 K outputs) 16.5 us against
+// 21.4, 400 x 400 (475 K) 35.6 against 38.4; 64 x 64^2 (738 K) 31.4 against 27.9, 512 x
+// 512 (780 K) 58.0 against 53.8, 16 x 256^2 (3.1 M) 151 against 108.
 constexpr long long kRhsAlone = 700000;
+
+// Waves from which a wave takes 2 x 2 or 2 x 1 tiles: two for every SIMD, all that
+// their registers leave room for.  Half the operand traffic, but half the waves.
+constexpr long long kWideTasks = 2048;
 
 static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
 {
@@ -979,9 +989,7 @@ static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
         rhs = *r;
         const long long outs = 3LL * rhs.M0 * rhs.M1 * rhs.batch;
         if (outs >= kRhsAlone) {
-            // many outputs: the tile form shares each row's y sums in LDS and runs
-            // by itself (64 x 256^2: 219 us; one output per thread 311)
-            rhs.rows_per_thread = 16;
+            rhs.rows_per_thread = 16;   // the tile form
             const int rc = pypde_rbc_rhs_banded(&rhs, s);
             if (rc != OK) return rc;
         } else {
@@ -989,12 +997,13 @@ static int phase1(const Stage& a, const pypde_rbc_rhs* r, hipStream_t s)
         }
     }
     const int HT = up((a.L0 + 1) / 2, 16);
-    // 2 x 2 tiles per wave (half the operand traffic) once they give every
-    // SIMD of the device two waves
+    // with the right-hand side, 2 x 2 / 2 x 1 / 1 x 1 tiles: 512 x 512 (1152 and 2304
+    // wide tasks) 58.9 / 52.6 / 55.0 us, 400 x 400 (780 and 1500) 49.8 / 41.4 / 34.3,
+    // 4 x 512^2 (4608 and 9216) 143 / 143 / 170
     const long long big = 3LL * a.batch * up(a.M1, 32) * 2 * up(HT, 2);
-    if (big >= 2048) {
+    if (big >= kWideTasks) {
         hipLaunchKernelGGL((stage_xpass<2, 2, 2>), dim3(nbr + blocks4(big)), dim3(256), 0, s, a, rhs, nbr, (int)big);
-    } else if (3LL * a.batch * up(a.M1, 16) * 2 * up(HT, 2) >= 2048) {
+    } else if (3LL * a.batch * up(a.M1, 16) * 2 * up(HT, 2) >= kWideTasks) {
         const long long t = 3LL * a.batch * up(a.M1, 16) * 2 * up(HT, 2);
         hipLaunchKernelGGL((stage_xpass<2, 1, 2>), dim3(nbr + blocks4(t)), dim3(256), 0, s, a, rhs, nbr, (int)t);
     } else {
@@ -1018,8 +1027,10 @@ static int phase2(const Stage& a, hipStream_t s)
 static int phase3(const Stage& a, hipStream_t s)
 {
     const int MT = up((a.M1 + 1) / 2, 16);
+    // 2 x 2 tiles against single ones: 576 tasks (512 x 512) 36.7 us against 32.4, 1152
+    // (8 x 256^2) 34.3 against 29.8, 2304 (16 x 256^2) 50.0 against 49.1
     const long long big = 3LL * a.batch * up(a.L0, 32) * up(MT, 2);
-    if (big >= 2048) {
+    if (big >= kWideTasks) {
         hipLaunchKernelGGL((stage_zconv<2, 2, 2>), dim3(blocks4(big)), dim3(256), 0, s, a, (int)big);
     } else {
         const long long t = 3LL * a.batch * up(a.L0, 16) * MT;
@@ -1042,8 +1053,9 @@ static int phase4_n(const Stage& a, hipStream_t s)
 template <int C>
 static int phase4_c(const Stage& a, hipStream_t s)
 {
-    // 32 columns per block once that still gives every CU two blocks (64 x 256^2: 152
-    // us against 226); the longest chains would spill registers in that form
+    // 32 columns per block once that still gives every CU two blocks (16 x 256^2, 768
+    // blocks: 40.0 us against 54.3 with 16; 256 x 256, 48: 15.8 against 10.5); the
+    // longest chains would spill registers in that form
     if constexpr (C < 16)
         if (6LL * a.batch * up(a.M1, 32) >= 512) return phase4_n<C, 2>(a, s);
     return phase4_n<C, 1>(a, s);
@@ -1058,7 +1070,8 @@ static int phase5_c(const Stage& a, hipStream_t s)
     if (const int rc = allow_lds<stage_hy<C>>(lds)) return rc;
     // four operator tiles per block while the blocks run side by side (two per CU,
     // one with the longest chains), else more, so that the solve is repeated less
-    // often (512 x 512: 800 blocks of four tiles 60 us)
+    // often (4, 8, 16 tiles: 256 x 256 10.6, 12.9, 18.5 us; 4 x 256^2 26.1, 21.3, 20.0;
+    // 512 x 512 61.4, 48.6, 37.9)
     int per = 4;
     while (per < 16 && (long long)rows * (up(kc, per) + up(kc + TN, per) + 1) > (C == 16 ? 256 : 512)) per *= 2;
     const int p0 = up(kc, per), p1 = up(kc + TN, per);
@@ -1080,8 +1093,10 @@ static int phase6_c(const Stage& a, hipStream_t s)
 static int phase7(const Stage& a, hipStream_t s)
 {
     const int T = 3 * up(a.M1, 16);
+    // 2 x 2 tiles against single ones: 768 tasks (512 x 512) 27.6 us against 24.1, 1536
+    // (8 x 256^2) 23.4 against 22.1, 3072 (16 x 256^2) 32.6 against 41.2
     const long long big = (long long)a.batch * up(a.M0, 32) * up(T, 2);
-    if (big >= 2048) {
+    if (big >= kWideTasks) {
         hipLaunchKernelGGL((stage_qy<2, 2, 2>), dim3(blocks4(big)), dim3(256), 0, s, a, (int)big);
     } else {
         const long long t = (long long)a.batch * up(a.M0, 16) * T;
@@ -1095,8 +1110,10 @@ static int phase8(const Stage& a, hipStream_t s)
     const long long pr = ((long long)a.N0 * a.N1 * a.batch + 255) / 256;
     const unsigned nbr = (unsigned)std::min<long long>(pr, 16384);
     const long long per = 4LL * a.batch * up((a.M0 + 1) / 2, 16);
+    // 32 columns per wave against 16: 1024 tasks (512 x 512) 12.6 us against 13.3, 2048
+    // (8 x 256^2) 17.5 against 15.9, 4096 (16 x 256^2) 25.6 against 27.4
     const long long big = per * up(a.M1, 32);
-    if (big >= 2048) {
+    if (big >= kWideTasks) {
         hipLaunchKernelGGL((stage_correct<2, 3>), dim3(nbr + blocks4(big)), dim3(256), 0, s, a, nbr, (int)big);
     } else {
         const long long t = per * up(a.M1, 16);

@@ -4,7 +4,7 @@ navier/rbc2d.py:28-434).
 Same constructor (`NavierStokes(case, shape=, ra=, pr=, dt=, tsave=, dealias=,
 integrator=, beta=, aspect=)`), fields (T, U, V, P, pres with .vhat / .v),
 `update()`, `iterate()`, `eval_Nu()`.  The step runs on the fused engine
-(pypde_amd.engine.RBCBatch, 19 launches per stage, optionally replayed from a
+(pypde_amd.engine.RBCBatch, eight phases per stage, optionally replayed from a
 HIP graph) for both integrators and any beta; only RK3 or beta != 1 with an odd
 dealiased y length falls back to the reference's operation sequence on the
 drop-in GPU operators.
