@@ -385,7 +385,8 @@ int pypde_rbc_rhs_banded(const pypde_rbc_rhs* args, void* stream);
  * bds [8][M0]: diagonals -1, 1, 3, 5 of (B D S)_x and -2, 0, 2, 4 of (B S)_x; sn: the
  * potential's stencil sub-diagonals, M0 of x then M1 of y; dtbc [L0][L1].  Line
  * solves (see pypde_recurrence) as parity chains padded with zeros to 16 C positions,
- * C = 2, 4, 8 or 16, the smallest with 16 C >= (M + 1) / 2: hx, hy per E
+ * C = 2, 4, 8 or 16, the smallest with 16 C >= (M + 1) / 2, position c C + k of a
+ * chain at [k / 2][c][k % 2] (c < 16): hx, hy per E
  * [even | odd][LM | R | MU | NU][16 C]; prec [even | odd][LM | R | MU | NU][M1][16 C].
  * mdtb, idta, nu per instance.
  * Limits: 6 <= M0, M1 <= PYPDE_STAGE_MAX_MODES. */

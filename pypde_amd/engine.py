@@ -269,13 +269,14 @@ def pack_operator(A, tiles=None, chunks=None):
 
 def _chains(tab):
     """Line tables [..., 4, M] as parity chains [..., even | odd, 4, 16 C], zero-padded;
-    C = 2, 4, 8 or 16 positions on each of 16 lanes."""
+    C = 2, 4, 8 or 16 positions on each of 16 lanes, position c C + k at
+    [k / 2][c][k % 2]."""
     M = tab.shape[-1]
     C = next(c for c in (2, 4, 8, 16) if 16 * c >= (M + 1) // 2)
     out = tab.new_zeros(tab.shape[:-2] + (2, 4, 16 * C))
     for q in (0, 1):
         out[..., q, :, :(M + 1 - q) // 2] = tab[..., q::2]
-    return out
+    return out.unflatten(-1, (16, C // 2, 2)).transpose(-2, -3).flatten(-3)
 
 
 def _halves(A, flip=0):
