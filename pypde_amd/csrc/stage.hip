@@ -1056,7 +1056,7 @@ template <int C>
 static int phase4_c(const Stage& a, hipStream_t s)
 {
     // 32 columns per block once that still gives every CU two blocks (16 x 256^2, 768
-    // blocks: 40.0 us against 54.3 with 16; 256 x 256, 48: 15.8 against 10.5); the
+    // blocks: 39.0 us against 52.3 with 16; 256 x 256, 48: 15.4 against 10.0); the
     // longest chains would spill registers in that form
     if constexpr (C < 16)
         if (6LL * a.batch * up(a.M1, 32) >= 512) return phase4_n<C, 2>(a, s);
@@ -1072,8 +1072,8 @@ static int phase5_c(const Stage& a, hipStream_t s)
     if (const int rc = allow_lds<stage_hy<C>>(lds)) return rc;
     // four operator tiles per block while the blocks run side by side (two per CU,
     // one with the longest chains), else more, so that the solve is repeated less
-    // often (4, 8, 16 tiles: 256 x 256 10.6, 12.9, 18.5 us; 4 x 256^2 26.1, 21.3, 20.0;
-    // 512 x 512 61.4, 48.6, 37.9)
+    // often (4, 8, 16 tiles: 256 x 256 10.1, 12.4, 18.3 us; 4 x 256^2 24.2, 20.3, 19.8;
+    // 512 x 512 45.4, 40.7, 33.9)
     int per = 4;
     while (per < 16 && (long long)rows * (up(kc, per) + up(kc + TN, per) + 1) > (C == 16 ? 256 : 512)) per *= 2;
     const int p0 = up(kc, per), p1 = up(kc + TN, per);
