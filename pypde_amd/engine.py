@@ -14,8 +14,8 @@ reference's LU factors, in the launches of the products next to them.
 The step with one launch per operator (below, 17 or so launches; with
 group_launches some of them share one) remains for exact_solves, which also takes
 more than the 512 modes per axis that a phase's lines and the register recurrences
-hold, for fewer than 6 modes on an axis, and as the member launches of a
-persistent heterogeneous batch (group_launches=False).
+hold, and as the member launches of a persistent heterogeneous batch
+(group_launches=False).
 
 Data layout in HBM (float64, row-major):
   X    [B, 3, M0, M1]      Galerkin coefficients of U, V (ChebDirichlet^2) and
